@@ -806,41 +806,49 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, uint8_t (&r
     tl_mark(p.tl, p.tl_cap, 6);  // diagnostics build: hand-off done (not the last split)
     return;
   }
-  // Row weights of the splits, exp2(m_s - max) / l (l summed in split order), in LDS (the first
-  // ring, no longer read).  Up to 16 splits the (m, l) pairs are loaded once, all in flight
-  // together; more splits take a second pass.
-  float* wts = reinterpret_cast<float*>(&ring0[0][0]);  // [ROWS][kAttnMergeMax]
-  static_assert(kAttnWaves * SLOT >= 64 * kAttnMergeMax * 4, "split weights fit the first ring");
-  constexpr int kMergeBatch = 16;
+  // Row weights of the splits, exp2(m_s - max) / l (l summed in split order), in LDS (the rings,
+  // no longer read).  All (m, l) pairs are fetched by all threads, in flight together, and every
+  // row's thread then walks its splits in LDS: a row's thread fetching its own pairs beyond the
+  // first 16 splits waited for each load in turn (B = 1, q_len 5, context 65536, 31 splits: the
+  // launch's graph replay 59.9 -> 53.5 us; B = 8, q_len 9, context 4096, 4 splits: 37.0 -> 36.3).
+  constexpr int WST = kAttnMergeMax + 1;  // row stride: the rows' threads walk different banks
+  float* wts = reinterpret_cast<float*>(&ring0[0][0]);  // [ROWS][WST], m then the weight
+  float* lst = reinterpret_cast<float*>(&ring1[0][0]);  // [ROWS][WST], l
+  static_assert(kAttnWaves * SLOT >= 64 * WST * 4, "split statistics fit a ring");
+  {
+    constexpr int PI = (ROWS * kAttnMergeMax + NT - 1) / NT;  // pairs per thread at the most splits
+    float mv[PI], lv[PI];
+    static_for<0, PI>([&](auto ic) __attribute__((always_inline)) {
+      constexpr int i = decltype(ic)::value;
+      const int e = threadIdx.x + NT * i;  // (split, row), as they lie in memory
+      if (NT * i < n_active * ROWS) {      // workgroup-uniform
+        const float* src = mlpart + (prog_base * ROWS + min(e, n_active * ROWS - 1)) * 2;
+        mv[i] = collect(src);
+        lv[i] = collect(src + 1);
+      }
+    });
+    static_for<0, PI>([&](auto ic) __attribute__((always_inline)) {
+      constexpr int i = decltype(ic)::value;
+      const int e = threadIdx.x + NT * i;
+      if (e < n_active * ROWS) {
+        wts[(e % ROWS) * WST + e / ROWS] = mv[i];
+        lst[(e % ROWS) * WST + e / ROWS] = lv[i];
+      }
+    });
+  }
+  __syncthreads();
   if (threadIdx.x < ROWS) {
-    const int row = threadIdx.x;
-    float* wt = wts + row * kAttnMergeMax;
-    auto ml_at = [&](int sp) { return mlpart + ((prog_base + (sp < n_active ? sp : 0)) * ROWS + row) * 2; };
-    float mv[kMergeBatch], lv[kMergeBatch];
-#pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u) {
-      mv[u] = collect(ml_at(u));
-      lv[u] = collect(ml_at(u) + 1);
-    }
+    float* wt = wts + threadIdx.x * WST;
+    const float* ls = lst + threadIdx.x * WST;
     float mx = -INFINITY;
-#pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u)
-      if (u < n_active) mx = fmaxf(mx, mv[u]);
-    for (int sp = kMergeBatch; sp < n_active; ++sp) mx = fmaxf(mx, collect(ml_at(sp)));
+    for (int sp = 0; sp < n_active; ++sp) mx = fmaxf(mx, wt[sp]);
     const float mxs = (mx == -INFINITY) ? 0.f : mx;
     float l = 0.f;
-#pragma unroll
-    for (int u = 0; u < kMergeBatch; ++u)
-      if (u < n_active) {
-        const float wgt = fast_exp2(mv[u] - mxs);
-        wt[u] = wgt;
-        const float lw = wgt * lv[u];
-        l = (u == 0) ? lw : l + lw;
-      }
-    for (int sp = kMergeBatch; sp < n_active; ++sp) {
-      const float wgt = fast_exp2(collect(ml_at(sp)) - mxs);
+    for (int sp = 0; sp < n_active; ++sp) {
+      const float wgt = fast_exp2(wt[sp] - mxs);
       wt[sp] = wgt;
-      l += wgt * collect(ml_at(sp) + 1);
+      const float lw = wgt * ls[sp];
+      l = (sp == 0) ? lw : l + lw;
     }
     const float inv = (l == 0.f) ? 0.f : 1.f / l;
     for (int sp = 0; sp < n_active; ++sp) wt[sp] *= inv;
@@ -848,28 +856,34 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, uint8_t (&r
   __syncthreads();
   // O rows: sum over splits in split order of weight * partial O.  All of a thread's items'
   // loads of SB splits are in flight together.
-  constexpr int SB = ITEMS <= 2 ? 8 : (ITEMS <= 4 ? 4 : 2);  // at most 16 16-byte loads in flight per thread
+  auto sum_splits = [&](auto sbc) __attribute__((always_inline)) {
+    constexpr int SB = decltype(sbc)::value;
+    for (int s0m = 0; s0m < n_active; s0m += SB) {
+      v4i t[SB][ITEMS];
+#pragma unroll
+      for (int u = 0; u < SB; ++u)
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it) {
+          const int e = threadIdx.x + NT * it;
+          t[u][it] = collect16(ors, oob_unless(ivalid[it] && s0m + u < n_active,
+                                               (uint32_t)(((s0m + u) * ROWS * QPR + e) * 16)));
+        }
+#pragma unroll
+      for (int u = 0; u < SB; ++u)
+#pragma unroll
+        for (int it = 0; it < ITEMS; ++it)
+          if (ivalid[it] && s0m + u < n_active) {
+            const int e = threadIdx.x + NT * it;
+            o[it] += wts[(e / QPR) * WST + s0m + u] * __builtin_bit_cast(v4f, t[u][it]);
+          }
+    }
+  };
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) o[it] = v4f{0.f, 0.f, 0.f, 0.f};
-  for (int s0m = 0; s0m < n_active; s0m += SB) {
-    v4i t[SB][ITEMS];
-#pragma unroll
-    for (int u = 0; u < SB; ++u)
-#pragma unroll
-      for (int it = 0; it < ITEMS; ++it) {
-        const int e = threadIdx.x + NT * it;
-        t[u][it] = collect16(ors, oob_unless(ivalid[it] && s0m + u < n_active,
-                                             (uint32_t)(((s0m + u) * ROWS * QPR + e) * 16)));
-      }
-#pragma unroll
-    for (int u = 0; u < SB; ++u)
-#pragma unroll
-      for (int it = 0; it < ITEMS; ++it)
-        if (ivalid[it] && s0m + u < n_active) {
-          const int e = threadIdx.x + NT * it;
-          o[it] += wts[(e / QPR) * kAttnMergeMax + s0m + u] * __builtin_bit_cast(v4f, t[u][it]);
-        }
-  }
+  // At most 16 16-byte loads in flight per thread for a few splits, 32 for many.
+  constexpr int SB = ITEMS <= 2 ? 8 : (ITEMS <= 4 ? 4 : 2);
+  if (n_active <= SB) sum_splits(std::integral_constant<int, SB>{});
+  else sum_splits(std::integral_constant<int, 2 * SB>{});
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it)
     if (ivalid[it]) store_row4(threadIdx.x + NT * it, o[it]);

@@ -255,3 +255,19 @@ def test_attention_out_of_pool_page_ids(D_, PAGE, sdt):
     K.paged_attention(q, kc, vc, ks, vs, bt_bad, cl, ql, QPP=ql, plan=plan.attn, out=o3)
     torch.cuda.synchronize()
     assert torch.equal(o3, outs[ql]), "plan mode differs from eager"
+
+
+@pytest.mark.parametrize("n_splits, q_len, sdt", [(16, 1, torch.float32), (17, 9, torch.float16), (33, 16, torch.float32),
+                                                  (64, 9, torch.float32)])
+def test_attention_merge_of_many_splits(n_splits, q_len, sdt):
+    """The merge of up to 64 splits (shortest split of a long table: 3 units of 128 tokens), 1 to 4 row blocks."""
+    Hs, D_, ctx = 4, 128, [128 * 3 * n_splits - 5]
+    kc, vc, ks, vs, bt, cl = gen.paged_kv(1, ctx, 1, D_, seed=n_splits, scale_dtype=sdt)
+    q = gen.queries(1, q_len, Hs, D_, seed=n_splits + 1)
+    note(f"attn merge n_splits={n_splits} q_len={q_len} {sdt}")
+    out, _ = K.paged_attention(*(t.to(DEV) for t in (q, kc, vc, ks, vs, bt, cl)), q_len)
+    one, _ = K.paged_attention(*(t.to(DEV) for t in (q, kc, vc, ks, vs, bt, cl)), q_len, QPP=1)
+    torch.cuda.synchronize()
+    ref = O.paged_attention(q.numpy(), kc.numpy(), vc.numpy(), ks.numpy(), vs.numpy(), bt.numpy(), cl.numpy(), q_len)
+    check(out, ref, q_len, f"{n_splits} splits")
+    assert torch.equal(one, out), f"QPP=1 differs from fused at {n_splits} splits"
