@@ -269,6 +269,8 @@ __host__ __device__ inline int chunked_grid(int units, int m_chunks) { return un
 // trailing partial block runs its units' chunks back to back): the chunks of one channel tile
 // share blockIdx.x mod 8 -- the XCD the dispatcher deals them to -- and run at the same time, so
 // the weight lines the first chunk reads from memory reach the other chunks from that XCD's L2.
+// Chunk-major order does the same only where units is a multiple of 8 (W8A8, N = 10000, K = 3072,
+// 79 channel tiles: M = 100 18.6 -> 15.7 us, 400 26.8 -> 24.2, 517 31.4 -> 28.7).
 __device__ __forceinline__ bool interleaved_unit(int m_chunks, int units, int& mc, int& unit) {
   const int id = blockIdx.x;
   const int full = (units / 8) * 8;
