@@ -28,6 +28,8 @@ inline int fail(int code, const char* what) {
 
 // Flag in the `variant` of a GEMM resource query: the call ran with a plan (tile rules differ).
 constexpr int kAttrsPlan = 16;
+// ... or the tiles are for an explicit request (W8A8: no many-row tile, which none names).
+constexpr int kAttrsStreaming = 32;
 // Flag in the `variant` of an attention resource query: fp32 K/V scales (else fp16).
 constexpr int kAttrsScaleFp32 = 1 << 16;
 

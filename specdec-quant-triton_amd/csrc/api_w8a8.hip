@@ -4,6 +4,8 @@
 //   RK      direct-activation streaming kernel (w8a8_rk.hpp) for 16-row token tiles: weights
 //           and activations go straight from memory into MFMA operand registers.
 //   WS      weight streaming with LDS-staged activations (w8a8_ws.hpp) for deeper token tiles.
+//   DEEP    many token rows (prompt chunks): both operands staged in LDS (w8a8_deep.hpp); eager
+//           calls with automatic tiles on packed weights, where it is priced lower than WS.
 //   LEGACY  register-pipelined kernel with 16/8/4/1-byte loads (w8a8.hpp): any alignment.
 // RK and WS read the row-major weight or the packed K-step-major fragments and need 16-byte
 // aligned activation rows.  Weight layout 2 is the packed INT4 weight of W4A8 (INT4 weights on
@@ -18,6 +20,7 @@
 
 #include "api_common.hpp"
 #include "w8a8.hpp"
+#include "w8a8_deep.hpp"
 #include "w8a8_plan.hpp"
 #include "w8a8_tiles.hpp"
 
@@ -139,12 +142,14 @@ namespace {
 
 // kPlan: plan-mode launch holding the menu of RK / WS tilings (w8a8_plan.hpp), one per 16 rows
 // of the active M.
-enum Family { kRk = 1, kWs = 2, kLegacy = 3, kPlan = 4 };
+// kDeep: many token rows, both operands staged in LDS (w8a8_deep.hpp).
+enum Family { kRk = 1, kWs = 2, kLegacy = 3, kPlan = 4, kDeep = 5 };
 
 struct W8A8Cfg {
   int family, layout;
   int mt, rw, nw, vec, splits, k_range, n_tiles, m_chunks;
   int bn;         // channels per workgroup
+  int deep;       // kDeep: the many-row tile (DeepTile)
   int bnsel;      // RK/WS channel-width variant (0..3 for 16/32/64/128)
   size_t lds, ws_partials, ws_counters;
   const void* fn;
@@ -287,10 +292,74 @@ void w8a8_auto_tiles(int M, int N, int K, double wb, int bnsel_fixed, int splits
   *splits = best_s;
 }
 
+// Measured price (us) of a many-row launch of `tiles` tiles over K: a start and an end, and per
+// 128-byte chunk of K the time of a round of workgroups, by how many of them a CU holds.  Fitted
+// to 48-2048 rows x 3000-28672 channels x K 1024-14336 (within 10 % of each; the matrix cores'
+// clock falls under the load of full rounds, so a round of lone workgroups runs faster).
+double w8a8_deep_price(int tile, int layout, int M, int N, int K, int cus) {
+  const int64_t tiles = (int64_t)ceil_div(M, kDeepRows[tile]) * ceil_div(N, kDeepChannels[tile]);
+  double per = 0;
+  if (tile == kDeepMix) {
+    // Whole rounds of 256 x 256 tiles, then what is left as halves (if it is at most half a round).
+    const int64_t rest = tiles % cus;
+    per = 1.85 * (tiles / cus) + (rest == 0 ? 0 : 4 * rest <= cus ? 0.75 : 2 * rest <= cus ? 1.0 : 1.7);
+  } else {
+    // Workgroups per CU, and the chunk time with 1, 2, .. of them; full rounds in steady state.
+    const int occ = tile == kDeep128 ? 1 : (tile == kDeep128Pair && layout == 2 ? 3 : 2);
+    const double part[2][3] = {{0.33, 0.60, 0}, {0.63, 1.00, 0}}, part4[3] = {0.64, 0.93, 1.25};
+    const double* t = layout == 2 ? part4 : part[tile == kDeep64 ? 0 : 1];
+    const double full = tile == kDeep64 ? 0.66 : tile == kDeep128 ? 0.58 : layout == 2 ? 1.33 : 1.10;
+    const int64_t slots = (int64_t)cus * occ, rest = tiles % slots;
+    per = full * (tiles / slots);
+    if (rest > 0) per += tile == kDeep128 ? (tiles < slots ? 0.50 : 0.55) : t[(rest - 1) / cus];
+  }
+  return 4.5 + per * ceil_div(K, 128);
+}
+
+// Measured price (us) of the streaming kernel's tile past 64 rows: per K step of 64 bytes a round of
+// workgroups takes 0.04 us and 2.2 ns a row at 128 channels (fitted at 80-304 rows, where the LDS
+// reads of the activations bound it), four fifths of that at 64 and less below.
+double w8a8_stream_price(int M, int N, int K, double wb, int mt, int sel, int s, int cus) {
+  const int chunks = ceil_div(ceil_div(M, 16), mt), rows = mt * 16, bn = bn_of_sel(sel);
+  const int rounds = ceil_div(ceil_div(N, bn) * s * chunks, cus);
+  const double step = (0.04 + 0.0022 * rows) * (sel == 3 ? 1.0 : (sel == 2 ? 0.8 : 0.7));
+  double t = std::max(rounds * step * (4 * ceil_div(K, 256)) / s, N * wb * K / 6e6) + 4.5;
+  if (s > 1) t += 1.0 + (double)s * rows * chunks * N * 8 / 4e6;
+  return t;
+}
+
+// The many-row tile of an eager call, or -1 where the streaming tile (mt, sel, s) is priced lower.
+// Both sides of the line, measured (us, streaming / many-row): N = 10000, K = 3072: M = 64 12.7 /
+// 12.6, 100 15.7 / 15.3, 192 19.7 / 13.3, 300 24.4 / 18.2; N = 3072, K = 8192: M = 256 22.0 / 24.7,
+// 517 32.0 / 26.0; N = K = 4096: M = 517 22.9 / 21.1, 1024 31.7 / 22.6; N = 28672, K = 4096: M = 517
+// 93 / 88, 1024 174 / 120, 2048 376 / 218; N = 4096, K = 14336: M = 517 53.9 / 56.8, 2048 144 / 101;
+// INT4 weights, N = 27648, K = 5120: M = 144 34.8 / 38.8, 256 55.3 / 40.0, 1024 206 / 131.
+int w8a8_deep_tile(int layout, int M, int N, int K, int mt, int sel, int s) {
+  if (M <= 64 || layout == 0) return -1;
+  const int cus = device_cus();
+  double best = w8a8_stream_price(M, N, K, layout == 2 ? 0.5 : 1.0, mt, sel, s, cus);
+  int tile = -1;
+  for (int i = 0; i < kDeepTiles; ++i) {
+    if (w8a8_deep_fn(i, layout) == nullptr) continue;
+    const double t = w8a8_deep_price(i, layout, M, N, K, cus);
+    if (t < best) { best = t; tile = i; }
+  }
+  return tile;
+}
+
+// Grid of a many-row launch and, of the mixed one, its whole tiles: every full round of them, and
+// a last round that fills more than half the CUs; the rest run as two halves each.
+int w8a8_deep_grid(const W8A8Cfg& cfg, int* whole) {
+  const int total = cfg.n_tiles * cfg.m_chunks, cus = device_cus(), rest = total % cus;
+  *whole = cfg.deep == kDeepMix && 2 * rest <= cus ? total - rest : total;
+  return *whole + 2 * (total - *whole);
+}
+
 // Resolve the kernel and its tiles.  `vec` is the operand alignment (16 when unknown),
-// `layout` 0 = row-major weight, 1 = packed fragments.
+// `layout` 0 = row-major weight, 1 = packed fragments.  `streaming`: no many-row tile (the answer is
+// one that explicit BLOCK_M, BLOCK_N and split_k name again).
 int w8a8_config(int layout, int m_grid, int N, int K, int block_m, int block_n, int num_warps, int split_k,
-                int vec, bool plan_mode, W8A8Cfg* cfg) {
+                int vec, bool plan_mode, bool streaming, W8A8Cfg* cfg) {
   SPECQ_REQUIRE(m_grid >= 0 && N > 0 && K > 0, SPECQ_EINVAL, "w8a8: bad sizes M=%d N=%d K=%d", m_grid, N, K);
   SPECQ_REQUIRE(block_n == 0 || block_n == 16 || block_n == 32 || block_n == 64 || block_n == 128, SPECQ_ENOTSUP,
                 "w8a8: BLOCK_N=%d must be 16, 32, 64 or 128", block_n);
@@ -318,6 +387,18 @@ int w8a8_config(int layout, int m_grid, int N, int K, int block_m, int block_n, 
     joint_splits = t_sk;
   } else if (joint) {
     w8a8_auto_tiles(m_grid, N, K, layout == 2 ? 0.5 : 1.0, want, split_k, &mt, &joint_sel, &joint_splits);
+    const int deep = block_n <= 0 && split_k <= 0 && !streaming
+                         ? w8a8_deep_tile(layout, m_grid, N, K, mt, joint_sel, joint_splits) : -1;
+    if (deep >= 0) {
+      cfg->family = kDeep; cfg->deep = deep; cfg->layout = layout; cfg->vec = vec; cfg->nw = 4; cfg->rw = 1;
+      cfg->fn = w8a8_deep_fn(deep, layout);
+      cfg->mt = kDeepRows[deep] / 16; cfg->bn = kDeepChannels[deep]; cfg->bnsel = 3;
+      cfg->n_tiles = ceil_div(N, cfg->bn);
+      cfg->m_chunks = ceil_div(m_grid, kDeepRows[deep]);
+      cfg->splits = 1; cfg->k_range = ceil_div(K, 256) * 256;
+      cfg->lds = cfg->ws_partials = cfg->ws_counters = 0;
+      return SPECQ_OK;
+    }
   } else if (block_m > 0) {
     SPECQ_REQUIRE(block_m % 16 == 0 && block_m <= 16 * kW8A8MaxMt, SPECQ_ENOTSUP,
                   "w8a8: BLOCK_M=%d must be a multiple of 16 and at most %d", block_m, 16 * kW8A8MaxMt);
@@ -568,8 +649,9 @@ int w8a8_plan_table(int m_grid, const W8A8Group& grp, int K, W8A8Cfg* cfg) {
 // Tiles of a grouped launch: chosen as for one GEMM of the members' total width, then every
 // member gets whole channel blocks of its own (its last block may be partial).
 int w8a8_group_config(int layout, int m_grid, const W8A8Group& grp, int K, int block_m, int block_n, int num_warps,
-                      int split_k, int vec, bool plan_mode, W8A8Cfg* cfg) {
-  int rc = w8a8_config(layout, m_grid, grp.n_total(), K, block_m, block_n, num_warps, split_k, vec, plan_mode, cfg);
+                      int split_k, int vec, bool plan_mode, W8A8Cfg* cfg, bool streaming = false) {
+  int rc = w8a8_config(layout, m_grid, grp.n_total(), K, block_m, block_n, num_warps, split_k, vec, plan_mode,
+                       streaming, cfg);
   if (rc) return rc;
   if (cfg->family == kPlan) return w8a8_plan_table(m_grid, grp, K, cfg);
   if (grp.n == 1) return rc;
@@ -655,7 +737,8 @@ int run_w8a8(int layout, const int8_t* a, int64_t lda, const W8A8Group& grp, con
       p.grp_vec_store[g - 1] = vec_store(grp.c[g], grp.ldc[g], grp.sw[g]);
     }
   }
-  const int grid = cfg.family == kPlan ? cfg.plan_grid : chunked_grid(cfg.n_tiles * cfg.splits, cfg.m_chunks);
+  int grid = cfg.family == kPlan ? cfg.plan_grid : chunked_grid(cfg.n_tiles * cfg.splits, cfg.m_chunks);
+  if (cfg.family == kDeep) grid = w8a8_deep_grid(cfg, &p.whole);
   if (static_scratch && need) {
     int n_ctr = cfg.family == kPlan ? cfg.n_counters : cfg.m_chunks * cfg.n_tiles;
     int32_t* ctr = p.counters;
@@ -713,11 +796,11 @@ size_t workspace_size(int layout, int m_grid, int N, int K, int block_m, int blo
 int w8a8_attrs(int layout, int m_grid, int N, int K, int block_m, int block_n, int num_warps, int split_k,
                specq_kernel_attrs* out) {
   W8A8Cfg cfg;
-  const bool plan_mode = (layout & kAttrsPlan) != 0;
-  layout &= ~kAttrsPlan;
+  const bool plan_mode = (layout & kAttrsPlan) != 0, streaming = (layout & kAttrsStreaming) != 0;
+  layout &= ~(kAttrsPlan | kAttrsStreaming);
   SPECQ_REQUIRE(layout >= 0 && layout <= 2, SPECQ_EINVAL, "w8a8 attrs: layout %d", layout);
   int rc = w8a8_group_config(layout, m_grid, single(nullptr, 0, nullptr, nullptr, 0, N), K, block_m, block_n,
-                             num_warps, split_k, 16, plan_mode, &cfg);
+                             num_warps, split_k, 16, plan_mode, &cfg, streaming);
   if (rc) return rc;
   hipFuncAttributes fa;
   if (hipFuncGetAttributes(&fa, cfg.fn) != hipSuccess) return fail(SPECQ_EIO, "w8a8: hipFuncGetAttributes failed");
@@ -727,6 +810,12 @@ int w8a8_attrs(int layout, int m_grid, int N, int K, int block_m, int block_n, i
   if (cfg.family == kPlan) {
     snprintf(out->name, sizeof(out->name), "specq::w8a8_plan_kernel<%d, %d>", cfg.layout,
              cfg.fn == (cfg.layout == 0 ? w8a8_plan_fn_l0(1) : (cfg.layout == 1 ? w8a8_plan_fn_l1(1) : w8a8_plan_fn_l2(1))));
+  } else if (cfg.family == kDeep) {
+    if (cfg.deep == kDeepMix)
+      snprintf(out->name, sizeof(out->name), "specq::w8a8_deep_mix_kernel<%d>", cfg.layout);
+    else
+      snprintf(out->name, sizeof(out->name), "specq::w8a8_deep_kernel<%d, 4, %d, %d>", kDeepRows[cfg.deep] / 32,
+               cfg.deep == kDeep64 ? 3 : (cfg.deep == kDeep128 ? 4 : 2), cfg.layout);
   } else if (cfg.family == kRk) {
     snprintf(out->name, sizeof(out->name), "specq::w8a8_rk_kernel<1, %d, %d, 4, %d>", rw, kw, cfg.layout);
   } else if (cfg.family == kWs) {
@@ -741,6 +830,8 @@ int w8a8_attrs(int layout, int m_grid, int N, int K, int block_m, int block_n, i
   out->scratch_bytes = (int)fa.localSizeBytes;
   out->threads = cfg.nw * 64;
   out->grid = cfg.family == kPlan ? cfg.plan_grid : chunked_grid(cfg.n_tiles * cfg.splits, cfg.m_chunks);
+  int whole;
+  if (cfg.family == kDeep) out->grid = w8a8_deep_grid(cfg, &whole);
   out->block_m = cfg.mt * 16; out->block_n = cfg.bn; out->num_warps = cfg.nw; out->split_k = cfg.splits;
   return SPECQ_OK;
 }

@@ -39,6 +39,7 @@ struct W8A8Params {
   int k_range;         // K bytes per split, a multiple of 64
   int32_t* partials;   // [m_chunks][n_tiles][splits][BM*BN] when splits > 1
   int32_t* counters;   // [m_chunks][n_tiles], zero between calls
+  int whole;           // many-row mixed launch: whole tiles ahead of the halved ones (w8a8_deep.hpp)
   int vec_store;       // 1 when C rows allow 8-byte aligned stores of 4 halves
   // Grouped launch: n_grp GEMMs that share A, sa, M and K (q, k and v; gate and up), each with
   // its own weight, channel scales, output and N.  Member 0 is W / ldw / sw / C / ldc / N above;

@@ -372,7 +372,7 @@ def w8a8_matmul(a_q, sa, w_q, sw, out=None, BLOCK_M=16, BLOCK_N=None, BLOCK_K=12
         if plan_tiles != "grid":
             raise RuntimeError(f"w8a8_matmul: plan_tiles={plan_tiles!r} (None or 'grid')")
         if not bm:
-            cfg = KernelInfo(0, 1 if packed else 0, m_grid, N, K, 0, bn, nw, split_k).config
+            cfg = KernelInfo(0, (1 if packed else 0) | 32, m_grid, N, K, 0, bn, nw, split_k).config
             bm, bn, split_k = cfg["block_m"], cfg["block_n"], cfg["split_k"]
     ws = workspace or _ws.shared(a_q.device)
     if packed:
@@ -455,7 +455,7 @@ def w8a8_matmul_grouped(a_q, sa, weights, outs=None, BLOCK_M=16, BLOCK_N=None, n
         if plan_tiles != "grid":
             raise RuntimeError(f"w8a8_matmul_grouped: plan_tiles={plan_tiles!r} (None or 'grid')")
         if not bm:
-            cfg = KernelInfo(0, layout, m_grid, N_total, K, 0, bn, nw, split_k).config
+            cfg = KernelInfo(0, layout | 32, m_grid, N_total, K, 0, bn, nw, split_k).config
             bm, bn, split_k = cfg["block_m"], cfg["block_n"], cfg["split_k"]
     arr = lambda ct, vals: (ct * n)(*vals)  # noqa: E731
     n_arr = arr(ctypes.c_int, Ns)

@@ -1,0 +1,93 @@
+"""The many-row W8A8 / W4A8 kernel (prompt chunks), which eager calls with automatic tiles run past
+64 rows: every tile it has, at ragged M, N and K, bit for bit against the formula in 64-bit sums
+(the INT32 sums are exact and the epilogue's roundings are fixed: fp32 after each scale, then fp16).
+"""
+import pytest
+import torch
+
+import kernels as K
+from gpu_util import note
+from specq import gen
+from specq.plan import Plan
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def operands(fmt, M, N, Kd, seed):
+    """(activations, token scales, packed weight, channel scales, the weight's integers)."""
+    a, sa = (t.to(DEV) for t in gen.w8a8_acts(M, Kd, seed=seed))
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    sw = torch.rand(N, device=DEV, generator=g) * 1e-3 + 1e-4
+    if fmt == "w8a8":
+        w = torch.randint(-127, 128, (N, Kd), dtype=torch.int8, device=DEV, generator=g)
+        return a, sa, K.pack_weight_int8(w), sw, w
+    q = torch.randint(0, 16, (N, Kd), dtype=torch.uint8, device=DEV, generator=g)
+    half = Kd // 2
+    return a, sa, K.pack_weight_w4a8((q[:, :half] | (q[:, half:] << 4)).contiguous()), sw, q.to(torch.int8) - 8
+
+
+def formula(a, sa, w, sw):
+    acc = (a.double() @ w.double().t()).float()
+    return ((acc * sa[:, None]) * sw[None, :]).half()
+
+
+# (format, M, N, K, kernel): one row past a tile, one short of it, odd N (unaligned output rows), K a
+# partial step, an odd number of steps, fewer steps than the ring holds.
+CASES = [
+    ("w8a8", 65, 10001, 3088, "deep_kernel<2, 4, 3, 1>"),
+    ("w8a8", 193, 7001, 1104, "deep_kernel<2, 4, 3, 1>"),
+    ("w8a8", 513, 3001, 1040, "deep_kernel<2, 4, 3, 1>"),
+    ("w8a8", 385, 7001, 1104, "deep_kernel<4, 4, 4, 1>"),
+    ("w8a8", 300, 10001, 3088, "deep_kernel<4, 4, 4, 1>"),
+    ("w8a8", 641, 10001, 3088, "deep_kernel<4, 4, 2, 1>"),
+    ("w8a8", 1281, 28673, 208, "deep_kernel<4, 4, 2, 1>"),
+    ("w8a8", 1281, 10001, 3088, "deep_mix_kernel<1>"),    # whole tiles only
+    ("w8a8", 1537, 28673, 1104, "deep_mix_kernel<1>"),    # three rounds of them, then halves
+    ("w8a8", 897, 15000, 144, "deep_mix_kernel<1>"),
+    ("w4a8", 700, 10001, 3088, "deep_kernel<4, 4, 2, 2>"),
+    ("w4a8", 193, 28673, 208, "deep_kernel<4, 4, 2, 2>"),
+    ("w4a8", 1023, 3001, 1040, "deep_kernel<4, 4, 2, 2>"),
+]
+
+
+@pytest.mark.parametrize("fmt, M, N, Kd, name", CASES)
+def test_many_rows_bit_exact(fmt, M, N, Kd, name):
+    note(f"{fmt} many rows M={M} N={N} K={Kd}")
+    a, sa, wp, sw, w = operands(fmt, M, N, Kd, seed=M)
+    mm = K.w8a8_matmul if fmt == "w8a8" else K.w4a8_matmul
+    big = torch.full((M + 3, N + 5), 7.0, dtype=torch.float16, device=DEV)
+    _, ck = mm(a, sa, wp, sw, out=big[:M, :N], BLOCK_M=None)
+    torch.cuda.synchronize()
+    assert name in ck.name, ck.name
+    assert torch.equal(big[:M, :N].view(torch.int16), formula(a, sa, w, sw).view(torch.int16)), ck.name
+    assert bool((big[M:] == 7.0).all()) and bool((big[:, N:] == 7.0).all()), "stored past M or N"
+
+
+def test_many_rows_grouped_members():
+    """Members whose widths are no whole tiles, one below a tile, on a strided activation."""
+    M, Kd, Ns = 1400, 1104, (7001, 40, 5000, 3000)
+    note(f"grouped many rows M={M} N={Ns} K={Kd}")
+    ops = [operands("w8a8", M, N, Kd, seed=900 + i) for i, N in enumerate(Ns)]
+    wide = torch.zeros((M, Kd + 48), dtype=torch.int8, device=DEV)
+    wide[:, 16:16 + Kd] = ops[0][0]
+    outs, ck = K.w8a8_matmul_grouped(wide[:, 16:16 + Kd], ops[0][1], [(o[2], o[3]) for o in ops], BLOCK_M=None)
+    torch.cuda.synchronize()
+    assert "deep_" in ck.name, ck.name
+    for o, op in zip(outs, ops):
+        ref = formula(ops[0][0], ops[0][1], op[4], op[3])
+        assert torch.equal(o.view(torch.int16), ref.view(torch.int16)), op[2].N
+
+
+def test_plan_at_grid_tiles_of_many_rows():
+    """plan_tiles="grid" asks for tiles that can be named explicitly: same bits, no row past M written."""
+    M, N, Kd, active = 700, 7000, 1040, 601
+    note(f"plan grid tiles M={M} active={active}")
+    a, sa, wp, sw, w = operands("w8a8", M, N, Kd, seed=5)
+    plan = Plan(DEV)
+    plan.set(1, active)
+    out = torch.full((M, N), 7.0, dtype=torch.float16, device=DEV)
+    K.w8a8_matmul(a, sa, wp, sw, out=out, BLOCK_M=None, plan=plan.gemm, grid_m_max=M, plan_tiles="grid")
+    torch.cuda.synchronize()
+    assert torch.equal(out[:active].view(torch.int16), formula(a, sa, w, sw)[:active].view(torch.int16))
+    assert bool((out[active:] == 7.0).all())
