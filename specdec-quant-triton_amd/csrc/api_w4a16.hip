@@ -13,6 +13,7 @@
 
 #include "api_common.hpp"
 #include "w4a16_plan.hpp"
+#include "w4a16_deep.hpp"
 #include "w4a16_tiles.hpp"
 
 namespace specq {
@@ -63,7 +64,8 @@ namespace {
 
 // kW4Plan: plan-mode launch holding the menu of LDS-staged tilings (w4a16_plan.hpp), one per
 // 16 rows of the active M.
-enum W4Family { kW4Rk = 1, kW4Ws = 2, kW4Plan = 3 };
+// kW4Deep: many token rows, 128 x 128 tiles, no split hand-off (w4a16_deep.hpp).
+enum W4Family { kW4Rk = 1, kW4Ws = 2, kW4Plan = 3, kW4Deep = 4 };
 
 struct W4Cfg {
   int family, layout, mt, rw, splits, bps, n_tiles, m_chunks, units, grid, nblocks;
@@ -206,6 +208,32 @@ int w4_plan_config(int layout, int m_grid, int N, int K, int split_k, W4Cfg* cfg
   return SPECQ_OK;
 }
 
+// A many-row launch: one workgroup per tile sums every split, so it needs no partials.
+void w4_deep_launch(W4Cfg* cfg) {
+  cfg->fn = w4a16_deep_fn(cfg->layout);
+  cfg->units = cfg->n_tiles;
+  cfg->grid = cfg->n_tiles * cfg->m_chunks;
+  cfg->ws_partials = cfg->ws_counters = 0;
+}
+
+// Whether an eager call of several K splits runs the many-row kernel rather than the streaming tile
+// (mt, rw), by measured prices (us).  Many-row: per round of workgroups a start and an end, 2.45 us
+// per pair of K blocks and 0.5 us per split.  Streaming: the model above, whose error past 512 rows
+// is a fifth, and the splits' partial tiles written and read back at 3 TB/s; together they come out
+// up to a sixth high (290 to 1500 rows of nine layers), which the line allows for.  Both sides of it,
+// measured (streaming / many-row): N = K = 4096: M = 512 40 / 46, 700 59 / 46, 1024 85 / 50; N = 4096,
+// K = 14336: M = 512 81 / 134, 1024 188 / 144, 2048 343 / 278; N = 6144, K = 4096: M = 1024 86 / 88.
+bool w4_deep_wins(int M, int N, int K, int splits, int mt, int rw) {
+  if (M <= 256 || splits <= 1) return false;
+  const int cus = device_cus(), rows16 = ceil_div(M, 16);
+  const int chunks = splits * ceil_div(ceil_div(K / 128, splits), 2);
+  const int rounds = ceil_div(ceil_div(M, 128) * ceil_div(N, 128), cus);
+  const double deep = rounds * (chunks * 2.45 + 5.0 + 0.5 * splits);
+  const double ws = 1.2 * w4_model_time(rows16, N, K, splits, mt, rw, cus) +
+                    (double)splits * ceil_div(rows16, mt) * mt * 16 * N * 8 / 3e6;
+  return deep < 0.83 * ws;
+}
+
 int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, int split_k, bool plan_mode,
               W4Cfg* cfg, bool allow_menu = true) {
   SPECQ_REQUIRE(layout >= 0 && layout <= 2, SPECQ_EINVAL, "w4a16: unknown weight layout %d", layout);
@@ -238,6 +266,7 @@ int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, in
     rw = 2;  // 128-channel blocks keep wide N (the fused gate_up) to one workgroup per CU
   }
   int t_bm = 0, t_bn = 0, t_sk = 0;
+  bool deep = false;
   if (block_m <= 0 && block_n <= 0 && !plan_mode && tuned_tile(1, N, K, std::max(m_grid, 1), &t_bm, &t_bn, &t_sk)) {
     // A launch shape of the measured table: its tile (the split count still follows N and K).
     mt = t_bm / 16;
@@ -247,12 +276,14 @@ int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, in
     const int s_auto = std::min(split_k > 0 ? split_k : w4_auto_splits(N, nb), nb);
     const int s_eff = ceil_div(nb, ceil_div(nb, s_auto));
     w4_auto_tiles(m_grid, N, K, s_eff, block_n > 0 ? rw : 0, &mt, &rw);
+    deep = block_n <= 0 && g_w4a16_path.load() == 0 && w4_deep_wins(m_grid, N, K, s_eff, mt, rw);
+    if (deep) { mt = 8; rw = 2; }
   }
   // The LDS-staged kernel is the default at every depth (measured faster than the register
   // stream even for 16-row tiles on the Llama-3-8B linears); the register stream stays
   // selectable for tiles of up to 32 rows.
   const int path = g_w4a16_path.load();
-  const int family = (path == kW4Rk && mt <= kW4RkMaxMt) ? kW4Rk : kW4Ws;
+  const int family = deep ? kW4Deep : (path == kW4Rk && mt <= kW4RkMaxMt) ? kW4Rk : kW4Ws;
 
   cfg->family = family; cfg->layout = layout; cfg->mt = mt; cfg->rw = rw;
   cfg->nblocks = K / 128;
@@ -269,7 +300,9 @@ int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, in
   cfg->ws_counters = cfg->splits > 1 ? kCounterBytes : 0;
   SPECQ_REQUIRE((int64_t)cfg->m_chunks * cfg->n_tiles <= kMaxCounters, SPECQ_ENOTSUP,
                 "w4a16: %d x %d tiles exceed the counter region", cfg->m_chunks, cfg->n_tiles);
-  if (family == kW4Rk) {
+  if (family == kW4Deep) {
+    w4_deep_launch(cfg);
+  } else if (family == kW4Rk) {
     cfg->fn = w4a16_rk_fn(mt, rw, layout);
   } else {
     switch (layout) {
@@ -335,6 +368,7 @@ int w4_group_config(int layout, int m_grid, int n_members, const int* N, int K, 
   cfg->grid = chunked_grid(cfg->units, cfg->m_chunks);
   cfg->ws_partials = cfg->splits > 1 ? align_up((size_t)cfg->m_chunks * tiles * cfg->splits * BM * BN * 4, 256) : 0;
   cfg->ws_counters = cfg->splits > 1 ? kCounterBytes : 0;
+  if (cfg->family == kW4Deep) w4_deep_launch(cfg);
   SPECQ_REQUIRE((int64_t)cfg->m_chunks * tiles <= kMaxCounters, SPECQ_ENOTSUP,
                 "w4a16_grouped: %d x %d tiles exceed the counter region", cfg->m_chunks, tiles);
   return SPECQ_OK;
@@ -355,6 +389,8 @@ int w4a16_attrs(int layout, int m_grid, int N, int K, int block_m, int block_n, 
   // The name carries the template arguments exactly as profilers print the kernel symbol.
   if (cfg.family == kW4Plan)
     snprintf(out->name, sizeof(out->name), "specq::w4a16_plan_kernel<%d>", layout);
+  else if (cfg.family == kW4Deep)
+    snprintf(out->name, sizeof(out->name), "specq::w4a16_deep_kernel<%d>", layout);
   else if (cfg.family == kW4Rk)
     snprintf(out->name, sizeof(out->name), "specq::w4a16_rk_kernel<%d, %d, %d>", cfg.mt, cfg.rw, layout);
   else {

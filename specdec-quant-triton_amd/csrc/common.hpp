@@ -314,6 +314,40 @@ __device__ __forceinline__ void split_decode(int unit, int n_tiles, int splits, 
   split = r % splits;
 }
 
+// ---- Many-row GEMMs (w8a8_deep.hpp, w4a16_deep.hpp).
+// Position in tile order of workgroup `id` of a run of n: XCD id % 8 takes a contiguous part.
+__device__ __forceinline__ int deep_order(int id, int n) {
+  const int x = id & 7;
+  return x * (n / 8) + min(x, n % 8) + (id >> 3);
+}
+// Tile `idx` in tile order: M-chunks fastest, in blocks of 8.
+__device__ __forceinline__ void deep_tile_of(int idx, int m_chunks, int n_tiles, int& mc, int& tile) {
+  constexpr int MB = 8;
+  const int full = m_chunks / MB * MB * n_tiles;  // tiles of whole blocks of MB M-chunks
+  if (idx < full) {
+    const int blk = idx / (MB * n_tiles), r = idx - blk * (MB * n_tiles);
+    mc = blk * MB + r % MB;
+    tile = r / MB;
+  } else {
+    const int r = idx - full, mb = m_chunks % MB;
+    mc = m_chunks / MB * MB + r % mb;
+    tile = r / mb;
+  }
+}
+// One 1 KB LDS DMA: lane l's 16 bytes land at lds + 16 l (an LDS DMA reads M0 one wait state
+// after it is written, hence the s_nop).
+__device__ __forceinline__ void deep_dma(v4i rs, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
+               : "memory", "m0");
+}
+// Raw buffer resource over n bytes from base (none when n <= 0, at most 2^31).
+__device__ __forceinline__ v4i deep_rsrc(const void* base, int64_t n) {
+  const uint64_t a = (uint64_t)(uintptr_t)base;
+  const int64_t m = n < 0 ? 0 : (n > (int64_t)kOOB ? (int64_t)kOOB : n);
+  return v4i{uniform((int)(uint32_t)a), uniform((int)((uint32_t)(a >> 32) & 0xFFFFu)), uniform((int)(uint32_t)m),
+             kRsrcWord3};
+}
+
 __device__ __forceinline__ void wait_all_memory() {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __builtin_amdgcn_s_waitcnt(0);

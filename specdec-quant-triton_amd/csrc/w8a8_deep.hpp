@@ -56,39 +56,6 @@ struct W8A8DeepCfg {
   static_assert(NSL >= 2 && LDS <= 160 * 1024 && (NSL - 1) * PER <= 63, "tile");
 };
 
-// Position in tile order of workgroup `id` of a run of n: XCD id % 8 takes a contiguous part.
-__device__ __forceinline__ int deep_order(int id, int n) {
-  const int x = id & 7;
-  return x * (n / 8) + min(x, n % 8) + (id >> 3);
-}
-// Tile `idx` in tile order: M-chunks fastest, in blocks of 8.
-__device__ __forceinline__ void deep_tile_of(int idx, int m_chunks, int n_tiles, int& mc, int& tile) {
-  constexpr int MB = 8;
-  const int full = m_chunks / MB * MB * n_tiles;  // tiles of whole blocks of MB M-chunks
-  if (idx < full) {
-    const int blk = idx / (MB * n_tiles), r = idx - blk * (MB * n_tiles);
-    mc = blk * MB + r % MB;
-    tile = r / MB;
-  } else {
-    const int r = idx - full, mb = m_chunks % MB;
-    mc = m_chunks / MB * MB + r % mb;
-    tile = r / mb;
-  }
-}
-// One 1 KB LDS DMA: lane l's 16 bytes land at lds + 16 l (an LDS DMA reads M0 one wait state
-// after it is written, hence the s_nop).
-__device__ __forceinline__ void deep_dma(v4i rs, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
-               : "memory", "m0");
-}
-// Raw buffer resource over n bytes from base (none when n <= 0, at most 2^31).
-__device__ __forceinline__ v4i deep_rsrc(const void* base, int64_t n) {
-  const uint64_t a = (uint64_t)(uintptr_t)base;
-  const int64_t m = n < 0 ? 0 : (n > (int64_t)kOOB ? (int64_t)kOOB : n);
-  return v4i{uniform((int)(uint32_t)a), uniform((int)((uint32_t)(a >> 32) & 0xFFFFu)), uniform((int)(uint32_t)m),
-             kRsrcWord3};
-}
-
 // One 32 FM x 32 FN tile: rows m0.., channel tile `tile` (launch-wide) of BN channels.
 template <int FM, int FN, int NSL, int WL>
 __device__ __forceinline__ void w8a8_deep_body(W8A8Params p, uint8_t* lds, int m0, int tile, int M) {

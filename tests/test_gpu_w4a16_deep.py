@@ -1,0 +1,73 @@
+"""The many-row W4A16 kernel (prompt chunks) against the streaming kernel it stands in for, bit for
+bit (one fp32 summation order for every tile), and both against 64-bit sums.
+
+Tolerance of the latter: the fp32 sums of K products and the fp16 rounding of the output, 2^-11 of
+the value and K * 2^-24 of the sum of the products' magnitudes.
+"""
+import pytest
+import torch
+
+import kernels as K
+from gpu_util import note
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def operands(layout, M, N, Kd, group, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    a = torch.randn((M, Kd), device=DEV, generator=g).half()
+    q = torch.randint(0, 16, (N, Kd), dtype=torch.uint8, device=DEV, generator=g)
+    sc = (torch.rand((N, Kd // group), device=DEV, generator=g) * 0.02 + 0.002).half()
+    half = Kd // 2
+    u8 = (q[:, :half] | (q[:, half:] << 4)).contiguous()
+    wp = u8 if layout == "u8" else (K.pack_int4_i32(q) if layout == "i32" else K.pack_weight_int4(u8))
+    deq = ((q.half() - 8).view(N, -1, group) * sc[..., None]).view(N, Kd)
+    return a, wp, sc, deq
+
+
+# (layout, M, N, K, group, split_k): one row past a tile and one short, odd N, an odd number of K
+# blocks per stream and per split, a last split shorter than the others, one block in all.
+CASES = [
+    ("packed", 1024, 4096, 4096, 128, 0),
+    ("packed", 1023, 4090, 1920, 128, 4),
+    ("packed", 1023, 4001, 1664, 64, 5),
+    ("packed", 1023, 4090, 2176, 128, 3),
+    ("packed", 700, 4096, 4096, 4096, 0),
+    ("packed", 1023, 4096, 640, 128, 2),
+    ("i32", 895, 4100, 1792, 128, 4),
+    ("i32", 1023, 4090, 1408, 32, 3),
+    ("u8", 1000, 4096, 2304, 128, 4),
+    ("u8", 769, 4030, 1280, 16, 4),
+]
+
+
+@pytest.mark.parametrize("layout, M, N, Kd, group, split_k", CASES)
+def test_many_rows_bits_of_the_streaming_kernel(layout, M, N, Kd, group, split_k):
+    note(f"w4a16 many rows {layout} M={M} N={N} K={Kd} group={group} split_k={split_k}")
+    a, wp, sc, deq = operands(layout, M, N, Kd, group, seed=M)
+    big = torch.full((M + 3, N + 8), 7.0, dtype=torch.float16, device=DEV)
+    kw = dict(group=group, BLOCK_K=min(64, group), split_k=split_k)
+    _, ck = K.w4a16_matmul(a, wp, sc, out=big[:M, :N], BLOCK_M=None, **kw)
+    ws, ck2 = K.w4a16_matmul(a, wp, sc, BLOCK_M=128, **kw)
+    torch.cuda.synchronize()
+    assert "deep_kernel" in ck.name and "ws_kernel" in ck2.name, (ck.name, ck2.name)
+    assert torch.equal(big[:M, :N].view(torch.int16), ws.view(torch.int16)), ck.name
+    assert bool((big[M:] == 7.0).all()) and bool((big[:, N:] == 7.0).all()), "stored past M or N"
+    ref, mag = a.double() @ deq.double().t(), a.double().abs() @ deq.double().abs().t()
+    assert bool(((ws.double() - ref).abs() <= ref.abs() * 2.0 ** -11 + mag * Kd * 2.0 ** -24 + 1e-7).all())
+
+
+def test_many_rows_grouped_and_nonfinite_rows():
+    """Grouped members of unequal width; an activation row with Inf and NaN leaves the other rows alone."""
+    M, Kd, Ns = 1020, 4096, (2048, 1030, 900)
+    note(f"w4a16 grouped many rows M={M} N={Ns}")
+    ops = [operands("packed", M, N, Kd, 128, seed=70 + i) for i, N in enumerate(Ns)]
+    a = ops[0][0].clone()
+    a[5, 3], a[5, 700], a[1019, 4095] = float("inf"), float("nan"), float("inf")
+    outs, ck = K.w4a16_matmul_grouped(a, [(o[1], o[2]) for o in ops], split_k=4)
+    torch.cuda.synchronize()
+    assert "deep_kernel" in ck.name, ck.name
+    for o, op in zip(outs, ops):
+        ref, _ = K.w4a16_matmul(a, op[1], op[2], BLOCK_M=128, split_k=4)
+        assert torch.equal(o.view(torch.int16), ref.view(torch.int16))
