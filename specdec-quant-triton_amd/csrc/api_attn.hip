@@ -137,7 +137,8 @@ extern "C" int specq_paged_attn(const void* q, int64_t s_qb, int64_t s_qt, int64
   if (n_qc == 0) return SPECQ_OK;
   const int target = g_attn_target.load() > 0 ? g_attn_target.load() : device_cus();
   // Eager calls know the active sequences; a plan may activate as few as one.
-  const int ns = n_splits_for(max_pages, PAGE, (plan ? 1 : std::max(n_seqs, 1)) * H_KV, target);
+  const int ns = n_splits_for(max_pages, PAGE, plan ? H_KV : std::max(n_seqs, 1) * H_KV * attn_row_programs(q_len, G),
+                              target);
   const int64_t progs = (int64_t)B_grid * H_KV * n_qc;
   const int rows = rb * 16;
   size_t need = 0;
@@ -152,6 +153,7 @@ extern "C" int specq_paged_attn(const void* q, int64_t s_qb, int64_t s_qt, int64
   // the exact count for an eager call, the most any active count needs in plan mode.
   int64_t wgs = (int64_t)(plan ? B_grid : n_seqs) * H_KV * n_qc * ns;
   if (plan) {
+    // Active query tokens that fill one program cut a sequence finest; past that the cut gets coarser.
     wgs = 0;
     for (int s = 1; s <= B_grid; ++s)
       wgs = std::max(wgs, (int64_t)s * H_KV * n_qc * n_splits_for(max_pages, PAGE, s * H_KV, target));

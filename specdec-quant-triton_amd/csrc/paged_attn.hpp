@@ -95,8 +95,16 @@ constexpr int kAttnRing = 4;                        // LDS chunk slots per wave
 constexpr float kAttnLazyP = 64.f;
 constexpr int64_t kAttnMaxTokens = (int64_t)kAttnUnit * kAttnMaxUnits * kAttnMergeMax;  // 524288
 
+// Programs of 64 packed rows a (sequence, KV head) pair of q_len query tokens fills: what its work
+// counts for in the split length.  Verification steps fit one; a prompt chunk of 256 tokens at G = 4
+// is 16 programs, each of which would otherwise be cut as finely as a lone one (B = 2, context 4096:
+// 11 splits, 2816 workgroups of 3 chunks a wave).  Measured at H = 32, H_KV = 8, D = 128, QPP = 16:
+// 256 tokens behind 3840 149 -> 47 us, two ragged sequences of them 267 -> 72, 2 x 64 tokens at
+// context 4096 78 -> 34, 17 tokens (two programs) 30 -> 29.  It does not depend on QPP.
+__host__ __device__ inline int attn_row_programs(int q_len, int G) { return q_len * G > 64 ? (q_len * G + 63) / 64 : 1; }
+
 // 128-token units per split for a sequence of L tokens when `pairs` (sequence, KV head) pairs
-// are active and the device has `target` CUs.
+// (times their row programs) are active and the device has `target` CUs.
 __host__ __device__ inline int attn_split_units(int L, int pairs, int target) {
   const int n = L > 0 ? (L + kAttnUnit - 1) / kAttnUnit : 1;
   const int pr = pairs > 0 ? pairs : 1;
@@ -238,7 +246,7 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, uint8_t (&r
   // page ids of the split can be fetched together with the context length and Q: one memory
   // round trip before the first K/V DMA.
   const int cap = p.max_pages * p.PAGE;
-  const int split_tokens = kAttnUnit * attn_split_units(cap, n_seqs * p.H_KV, p.target_wgs);
+  const int split_tokens = kAttnUnit * attn_split_units(cap, n_seqs * p.H_KV * attn_row_programs(q_len, p.G), p.target_wgs);
   // The grid is one-dimensional: workgroup id = program * splits + split (the exception for
   // eager calls with several query chunks and long splits is below), with the split count
   // of the active sequences, so the workgroups that have work are the first ones dispatched and

@@ -271,3 +271,28 @@ def test_attention_merge_of_many_splits(n_splits, q_len, sdt):
     ref = O.paged_attention(q.numpy(), kc.numpy(), vc.numpy(), ks.numpy(), vs.numpy(), bt.numpy(), cl.numpy(), q_len)
     check(out, ref, q_len, f"{n_splits} splits")
     assert torch.equal(one, out), f"QPP=1 differs from fused at {n_splits} splits"
+
+
+@pytest.mark.parametrize("q_len, G, ctx", [(16, 4, [4100, 700]), (17, 4, [4100, 17]), (48, 2, [2500, 48]),
+                                           (130, 4, [1700, 131]), (9, 8, [5000, 9])])
+def test_attention_chunks_of_more_than_one_program(q_len, G, ctx):
+    """Prompt chunks: around 64 packed rows (one row program) and past it the split length changes with
+    q_len; QPP = 1, the largest QPP and a plan replay cut alike, and the last chunk may be partial."""
+    B, Hkv, D_ = len(ctx), 2, 128
+    kc, vc, ks, vs, bt, cl = gen.paged_kv(B, ctx, Hkv, D_, seed=q_len)
+    q = gen.queries(B, q_len, Hkv * G, D_, seed=q_len + 1)
+    note(f"attn chunk q_len={q_len} G={G} ctx={ctx}")
+    args = [t.to(DEV) for t in (q, kc, vc, ks, vs, bt, cl)]
+    qpp = 64 // G
+    out, _ = K.paged_attention(*args, q_len, QPP=qpp)
+    one, _ = K.paged_attention(*args, q_len, QPP=1)
+    plan = torch.tensor([B, q_len], dtype=torch.int32, device=DEV)
+    wide = torch.zeros((B, q_len + 3, Hkv * G, D_), dtype=torch.float16, device=DEV)
+    wide[:, :q_len] = args[0]
+    planned, _ = K.paged_attention(wide, *args[1:], q_len + 3, QPP=qpp, plan=plan)
+    torch.cuda.synchronize()
+    ref = O.paged_attention(*(t.numpy() for t in (q, kc, vc, ks, vs, bt, cl)), q_len)
+    check(out, ref, q_len, f"chunk q_len={q_len}")
+    assert torch.equal(one, out), "QPP=1 differs"
+    assert torch.equal(planned[:, :q_len], out), "plan differs"
+    assert bool((planned[:, q_len:] == 0).all())
