@@ -316,7 +316,7 @@ double w8a8_deep_price(int tile, int layout, int M, int N, int K, int cus) {
   return 4.5 + per * ceil_div(K, 128);
 }
 
-// Measured price (us) of the streaming kernel's tile past 64 rows: per K step of 64 bytes a round of
+// Measured price (us) of the streaming kernel's tile past 128 rows: per K step of 64 bytes a round of
 // workgroups takes 0.04 us and 2.2 ns a row at 128 channels (fitted at 80-304 rows, where the LDS
 // reads of the activations bound it), four fifths of that at 64 and less below.
 double w8a8_stream_price(int M, int N, int K, double wb, int mt, int sel, int s, int cus) {
@@ -329,13 +329,13 @@ double w8a8_stream_price(int M, int N, int K, double wb, int mt, int sel, int s,
 }
 
 // The many-row tile of an eager call, or -1 where the streaming tile (mt, sel, s) is priced lower.
-// Both sides of the line, measured (us, streaming / many-row): N = 10000, K = 3072: M = 64 12.7 /
-// 12.6, 100 15.7 / 15.3, 192 19.7 / 13.3, 300 24.4 / 18.2; N = 3072, K = 8192: M = 256 22.0 / 24.7,
+// Both sides of the line, measured (us, streaming / many-row): N = 10240, K = 3072: M = 72 12.1 /
+// 13.9; N = 10000, K = 3072: M = 100 15.7 / 15.3, 192 19.7 / 13.3, 300 24.4 / 18.2; N = 3072, K = 8192: M = 256 22.0 / 24.7,
 // 517 32.0 / 26.0; N = K = 4096: M = 517 22.9 / 21.1, 1024 31.7 / 22.6; N = 28672, K = 4096: M = 517
 // 93 / 88, 1024 174 / 120, 2048 376 / 218; N = 4096, K = 14336: M = 517 53.9 / 56.8, 2048 144 / 101;
 // INT4 weights, N = 27648, K = 5120: M = 144 34.8 / 38.8, 256 55.3 / 40.0, 1024 206 / 131.
 int w8a8_deep_tile(int layout, int M, int N, int K, int mt, int sel, int s) {
-  if (M <= 64 || layout == 0) return -1;
+  if (M <= 128 || layout == 0) return -1;
   const int cus = device_cus();
   double best = w8a8_stream_price(M, N, K, layout == 2 ? 0.5 : 1.0, mt, sel, s, cus);
   int tile = -1;
