@@ -181,10 +181,17 @@ __device__ __forceinline__ v4i attn_rsrc(const void* base) {
   const uint64_t a = (uint64_t)(uintptr_t)base;
   return v4i{(int)(uint32_t)a, (int)((uint32_t)(a >> 32) & 0xFFFFu), (int)kOOB, kRsrcWord3};
 }
+// NT: the line is not kept in L2 (non-temporal).
+template <bool NT>
 __device__ __forceinline__ void dma16_rs(v4i rs, uint32_t voff, uint8_t* lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs),
-               "s"(lds_addr(lds))
-               : "memory", "m0");
+  if constexpr (NT)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen nt lds" ::"v"(voff), "s"(rs),
+                 "s"(lds_addr(lds))
+                 : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs),
+                 "s"(lds_addr(lds))
+                 : "memory", "m0");
 }
 __device__ __forceinline__ void dma4_global(const void* src, uint8_t* lds) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds_addr(lds)) : "memory", "m0");
@@ -394,6 +401,11 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, uint8_t (&r
     kv_base_v = (int64_t)pg * p.s_kp + (int64_t)tk * p.s_ko + (int64_t)kvh * p.s_kh;
     sc_base_v = ((int64_t)pg * p.s_sp + (int64_t)tk * p.s_so + (int64_t)kvh * p.s_sh) * (int64_t)sizeof(ST);
   }
+  // One query chunk: no other program reads these K/V bytes, and keeping them out of L2 leaves the
+  // lines of scales there, which the sequence's KV heads share (B = 32, one token, context 8192 116 ->
+  // 111 us, 4096 63.6 -> 60.8; B = 1, q_len 5, context 65536 45.1 -> 42.6).  Several query chunks read
+  // them again from L2 (2 x 256 tokens at context 4096: 70.0 us, and 71.7 kept out of it).
+  const bool read_once = p.n_qc == 1;
   // Issue the DMAs of chunk `it` into ring slot SL.  K/V granules of chunks past the wave's
   // last or on a page outside the pool, and of tokens at or past kv_end, are out of range
   // (zeros); their scales read a fixed valid address.
@@ -406,10 +418,17 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, uint8_t (&r
     const int64_t sb = readlane64(sc_base_v, li);
     const v4i rk = attn_rsrc(p.kc + kb), rv = attn_rsrc(p.vc + kb);
     if (real && t0 + kAttnChunk <= kv_end) {
+      if (read_once) {
 #pragma unroll
-      for (int i = 0; i < NDMA; ++i) dma16_rs(rk, kvoff[i], dst + 1024 * i);
+        for (int i = 0; i < NDMA; ++i) dma16_rs<true>(rk, kvoff[i], dst + 1024 * i);
 #pragma unroll
-      for (int i = 0; i < NDMA; ++i) dma16_rs(rv, kvoff[i], dst + KB + 1024 * i);
+        for (int i = 0; i < NDMA; ++i) dma16_rs<true>(rv, kvoff[i], dst + KB + 1024 * i);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NDMA; ++i) dma16_rs<false>(rk, kvoff[i], dst + 1024 * i);
+#pragma unroll
+        for (int i = 0; i < NDMA; ++i) dma16_rs<false>(rv, kvoff[i], dst + KB + 1024 * i);
+      }
       const uint8_t* src = sc_lane + sb;
       if constexpr (sizeof(ST) == 4) dma4_global(src, dst + SC);
       else dma2_global(src, dst + SC);
@@ -417,12 +436,12 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, uint8_t (&r
 #pragma unroll
       for (int i = 0; i < NDMA; ++i) {
         const bool ok = real && t0 + (64 * i + lane) / GR < kv_end;
-        dma16_rs(rk, oob_unless(ok, kvoff[i]), dst + 1024 * i);
+        dma16_rs<false>(rk, oob_unless(ok, kvoff[i]), dst + 1024 * i);
       }
 #pragma unroll
       for (int i = 0; i < NDMA; ++i) {
         const bool ok = real && t0 + (64 * i + lane) / GR < kv_end;
-        dma16_rs(rv, oob_unless(ok, kvoff[i]), dst + KB + 1024 * i);
+        dma16_rs<false>(rv, oob_unless(ok, kvoff[i]), dst + KB + 1024 * i);
       }
       const bool ok = real && t0 + sc_T < kv_end;
       const uint8_t* src = ok ? sc_lane + sb : sc_src;
