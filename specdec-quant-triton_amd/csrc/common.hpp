@@ -340,10 +340,10 @@ __device__ __forceinline__ void deep_dma(v4i rs, uint32_t voff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
                : "memory", "m0");
 }
-// Raw buffer resource over n bytes from base (none when n <= 0, at most 2^31).
+// Raw buffer resource over n bytes from base (none when n <= 0, at most 2^32 - 1: offsets are unsigned).
 __device__ __forceinline__ v4i deep_rsrc(const void* base, int64_t n) {
   const uint64_t a = (uint64_t)(uintptr_t)base;
-  const int64_t m = n < 0 ? 0 : (n > (int64_t)kOOB ? (int64_t)kOOB : n);
+  const int64_t m = n < 0 ? 0 : (n > 0xFFFFFFFFll ? 0xFFFFFFFFll : n);
   return v4i{uniform((int)(uint32_t)a), uniform((int)((uint32_t)(a >> 32) & 0xFFFFu)), uniform((int)(uint32_t)m),
              kRsrcWord3};
 }

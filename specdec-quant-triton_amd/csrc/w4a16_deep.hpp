@@ -76,7 +76,7 @@ __global__ __launch_bounds__(512) void w4a16_deep_kernel(W4A16Params p) {
 #pragma unroll
   for (int i = 0; i < A_L; ++i) {
     const int row = 4 * (w * A_L + i) + g, c = r ^ (row & 15);
-    a_off[i] = (uint32_t)(row * (int)p.lda * 2 + (LAYOUT == 0 ? (c < 8 ? 16 * c : p.K + 16 * (c - 8)) : 16 * c));
+    a_off[i] = (uint32_t)row * (uint32_t)p.lda * 2 + (LAYOUT == 0 ? (c < 8 ? 16 * c : p.K + 16 * (c - 8)) : 16 * c);
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds + (uint32_t)(h * 2 * SLOT + w * A_L * 1024);
   auto dma = [&](const Cursor& c, int slot) __attribute__((always_inline)) {

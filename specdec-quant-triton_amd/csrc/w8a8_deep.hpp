@@ -79,7 +79,7 @@ __device__ __forceinline__ void w8a8_deep_body(W8A8Params p, uint8_t* lds, int m
 #pragma unroll
   for (int i = 0; i < C::A_L; ++i) {
     const int row = 8 * (w * C::A_L + i) + (lane >> 3);
-    a_off[i] = (uint32_t)(row * (int)p.lda + 16 * ((lane & 7) ^ ((row >> 1) & 7)));
+    a_off[i] = (uint32_t)row * (uint32_t)p.lda + 16 * ((lane & 7) ^ ((row >> 1) & 7));
   }
 #pragma unroll
   for (int i = 0; i < C::W_L; ++i) {

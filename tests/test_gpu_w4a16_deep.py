@@ -71,3 +71,17 @@ def test_many_rows_grouped_and_nonfinite_rows():
     for o, op in zip(outs, ops):
         ref, _ = K.w4a16_matmul(a, op[1], op[2], BLOCK_M=128, split_k=4)
         assert torch.equal(o.view(torch.int16), ref.view(torch.int16))
+
+
+def test_many_rows_over_wide_strides():
+    """Activation rows that span more than 2 GiB within a tile: every row is read where it lies."""
+    M, N, Kd, ld = 700, 4096, 4096, 12 << 20
+    note(f"w4a16 many rows M={M} lda={ld}")
+    a, wp, sc, _ = operands("packed", M, N, Kd, 128, seed=6)
+    wide = torch.empty((M, ld), dtype=torch.float16, device=DEV)
+    wide[:, :Kd] = a
+    out, ck = K.w4a16_matmul(wide[:, :Kd], wp, sc, BLOCK_M=None)
+    ref, _ = K.w4a16_matmul(a, wp, sc, BLOCK_M=128)
+    torch.cuda.synchronize()
+    assert "deep_kernel" in ck.name, ck.name
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16))

@@ -91,3 +91,16 @@ def test_plan_at_grid_tiles_of_many_rows():
     torch.cuda.synchronize()
     assert torch.equal(out[:active].view(torch.int16), formula(a, sa, w, sw)[:active].view(torch.int16))
     assert bool((out[active:] == 7.0).all())
+
+
+def test_many_rows_over_wide_strides():
+    """Activation rows that span more than 2 GiB within a tile: every row is read where it lies."""
+    M, N, Kd, ld = 193, 7001, 1104, 40 << 20
+    note(f"w8a8 many rows M={M} lda={ld}")
+    a, sa, wp, sw, w = operands("w8a8", M, N, Kd, seed=6)
+    wide = torch.empty((M, ld), dtype=torch.int8, device=DEV)
+    wide[:, :Kd] = a
+    out, ck = K.w8a8_matmul(wide[:, :Kd], sa, wp, sw, BLOCK_M=None)
+    torch.cuda.synchronize()
+    assert "deep_kernel<2, 4, 3, 1>" in ck.name, ck.name
+    assert torch.equal(out.view(torch.int16), formula(a, sa, w, sw).view(torch.int16)), ck.name
