@@ -69,6 +69,7 @@ enum W4Family { kW4Rk = 1, kW4Ws = 2, kW4Plan = 3, kW4Deep = 4 };
 
 struct W4Cfg {
   int family, layout, mt, rw, splits, bps, n_tiles, m_chunks, units, grid, nblocks;
+  bool keep = false;  // kW4Ws: weights stay in L2 for the other M-chunks
   size_t ws_partials, ws_counters;
   const void* fn;
   W4PlanTile plan_t[kW4PlanRows];  // kW4Plan: the tiling of each 16-row step of M
@@ -305,10 +306,14 @@ int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, in
   } else if (family == kW4Rk) {
     cfg->fn = w4a16_rk_fn(mt, rw, layout);
   } else {
+    // Weights that several M-chunks read stay in L2 (N = 4096, K = 14336: M = 512 81.5 -> 78.6 us;
+    // N = 28672, K = 4096: M = 288 79.2 -> 75.9, 1024 293 -> 288); with one chunk they are read once and
+    // do not (a layer's four launches at M = 72: 79 us, and 84 kept).
+    cfg->keep = !plan_mode && cfg->m_chunks > 1 && mt >= kW4KeepMt;
     switch (layout) {
-      case 0: cfg->fn = w4a16_ws_fn_l0(mt, rw); break;
-      case 1: cfg->fn = w4a16_ws_fn_l1(mt, rw); break;
-      default: cfg->fn = w4a16_ws_fn_l2(mt, rw); break;
+      case 0: cfg->fn = w4a16_ws_fn_l0(mt, rw, cfg->keep); break;
+      case 1: cfg->fn = w4a16_ws_fn_l1(mt, rw, cfg->keep); break;
+      default: cfg->fn = w4a16_ws_fn_l2(mt, rw, cfg->keep); break;
     }
   }
   SPECQ_REQUIRE(cfg->fn != nullptr, SPECQ_ENOTSUP, "w4a16: no kernel for BLOCK_M=%d BLOCK_N=%d", mt * 16, 64 * rw);
@@ -396,7 +401,7 @@ int w4a16_attrs(int layout, int m_grid, int N, int K, int block_m, int block_n, 
   else {
     int s = 0, nslot = 0, nsw = 0;
     w4a16_ws_shape(cfg.mt, cfg.rw, layout, &s, &nslot, &nsw);
-    snprintf(out->name, sizeof(out->name), "specq::w4a16_ws_kernel<%d, %d, %d, %d, %d, %d>", cfg.mt, cfg.rw, s,
+    snprintf(out->name, sizeof(out->name), "specq::w4a16_%sws_kernel<%d, %d, %d, %d, %d, %d>", cfg.keep ? "chunks_" : "", cfg.mt, cfg.rw, s,
              nslot, nsw, layout);
   }
   out->num_regs = fa.numRegs;

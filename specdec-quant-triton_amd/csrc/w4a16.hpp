@@ -167,7 +167,8 @@ template <int LAYOUT>
 struct W4Nsc { static constexpr int value = LAYOUT == 0 ? 2 : 1; };
 
 // Per-wave weight and scale addressing for RW 16-row fragments starting at channel n0.
-template <int RW, int LAYOUT>
+// KEEP: the weight lines stay in L2 for the other workgroups that read them.
+template <int RW, int LAYOUT, bool KEEP = false>
 struct W4Weights {
   static constexpr int NSC = W4Nsc<LAYOUT>::value;
   rsrc_t wsrc, ssrc;
@@ -204,13 +205,14 @@ struct W4Weights {
 #pragma unroll
     for (int i = 0; i < RW; ++i) srow[i] = (16 * i + r < rows_w) ? (int32_t)((16 * i + r) * p.ld_sc + sadj) : -1;
   }
-  // Loads of block b (live: inside this wave's range).  NT loads: the weight is streamed once.
+  // Loads of block b (live: inside this wave's range).  NT loads unless other
+  // M-chunks read the weight too.
   __device__ __forceinline__ void issue(int b, bool live, v4i (&wv)[RW], uint32_t (&sv)[RW][NSC]) const {
 #pragma unroll
     for (int i = 0; i < RW; ++i) {
       const bool ok = live & (wrow[i] != kOOB);
       const bool oks = live & (srow[i] >= 0);
-      wv[i] = __builtin_amdgcn_raw_buffer_load_b128(wsrc, oob_unless(ok, wrow[i] + (uint32_t)b * bstride), 0, 2);
+      wv[i] = __builtin_amdgcn_raw_buffer_load_b128(wsrc, oob_unless(ok, wrow[i] + (uint32_t)b * bstride), 0, KEEP ? 0 : 2);
 #pragma unroll
       for (int h = 0; h < NSC; ++h) {
         const int e = srow[i] + (w4_k<LAYOUT>(b, 2 * h, g, halfK) >> gshift);

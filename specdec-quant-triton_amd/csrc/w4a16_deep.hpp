@@ -13,7 +13,8 @@
 // workgroup adds them, with nothing handed over.
 //
 // Measured (us, streaming -> here): M = 1024, N = K = 4096 85 -> 50, N = 4096, K = 14336 188 -> 144,
-// M = 1500, N = K = 5120 134 -> 106.  Unsplit layers stay with the streaming kernel, which runs them at
+// M = 1500, N = K = 5120 134 -> 106; with the weight loads kept in L2, where the other M-chunks of the
+// channel tile find them, instead of non-temporal, M = 1024, K = 14336 142 -> 134, 700 126 -> 117.  Unsplit layers stay with the streaming kernel, which runs them at
 // the same rate (0.75 to 0.85 PFLOP/s).  Copies without the dequantization, without the LDS reads and
 // without the DMAs ran within a few percent of the kernel.  Also tried: the next fragment
 // dequantized between the MFMAs of this one, wave priorities by stream and around the MFMAs, weights
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(512) void w4a16_deep_kernel(W4A16Params p) {
     for (int t = 0; t < FM; ++t) af[t] = *reinterpret_cast<const v8h*>(a_rd + slot * SLOT + t * 4096 + pc[u]);
   };
 
-  W4Weights<FN, LAYOUT> wt;
+  W4Weights<FN, LAYOUT, true> wt;  // read by every M-chunk
   wt.init(p, n0);
   v4i wq[NW][FN];
   uint32_t sv[NW][FN][NSC];

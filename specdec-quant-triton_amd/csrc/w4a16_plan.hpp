@@ -40,7 +40,7 @@ __device__ __forceinline__ void w4a16_plan_path(const W4A16Params& p, SlotPtr sl
   static_assert(P::Cfg::SLOT <= kW4PlanSlotA && (P::NSLOT <= 2 || P::Cfg::SLOT <= kW4PlanSlotB) && P::NSLOT <= 4 &&
                     4 * RW * MT * 1024 <= 2 * kW4PlanSlotA,
                 "menu tiling fits the shared slots");
-  w4a16_ws_body<MT, RW, P::S, P::NSLOT, P::NSW, LAYOUT>(p, slots);
+  w4a16_ws_body<MT, RW, P::S, P::NSLOT, P::NSW, LAYOUT, false>(p, slots);
 }
 
 template <int LAYOUT>

@@ -12,6 +12,9 @@ namespace specq {
 
 constexpr int kW4MaxMt = 10;    // deepest token tile (160 rows: two streams x two 40 KB LDS slots = 160 KB)
 constexpr int kW4RkMaxMt = 2;
+// Token tiles from 80 rows up, which automatic tiles give several M-chunks, also come with weight
+// loads that stay in L2 (w4a16_chunks_ws_kernel), for launches that have them.
+constexpr int kW4KeepMt = 5;
 
 // LDS ring and weight-ring depth per tile (measured on the Llama-3-8B linears, 8-wave
 // kernel): chunks of 2 blocks for 16-row tiles (1 beyond), 2 LDS slots per stream (one chunk
@@ -28,8 +31,11 @@ struct W4WsPick {
 int w4a16_ws_shape(int mt, int rw, int layout, int* s, int* nslot, int* nsw);
 
 template <int MT, int RW, int LAYOUT>
-const void* w4a16_ws_pick() {
+const void* w4a16_ws_pick(bool keep) {
   using P = W4WsPick<MT, RW, LAYOUT>;
+  if constexpr (MT >= kW4KeepMt) {
+    if (keep) return reinterpret_cast<const void*>(&w4a16_chunks_ws_kernel<MT, RW, P::S, P::NSLOT, P::NSW, LAYOUT>);
+  }
   return reinterpret_cast<const void*>(&w4a16_ws_kernel<MT, RW, P::S, P::NSLOT, P::NSW, LAYOUT>);
 }
 template <int MT, int RW, int LAYOUT>
@@ -38,9 +44,9 @@ const void* w4a16_rk_pick() {
 }
 
 // Defined in the instantiation units.
-const void* w4a16_ws_fn_l0(int mt, int rw);
-const void* w4a16_ws_fn_l1(int mt, int rw);
-const void* w4a16_ws_fn_l2(int mt, int rw);
+const void* w4a16_ws_fn_l0(int mt, int rw, bool keep);
+const void* w4a16_ws_fn_l1(int mt, int rw, bool keep);
+const void* w4a16_ws_fn_l2(int mt, int rw, bool keep);
 const void* w4a16_rk_fn(int mt, int rw, int layout);
 
 }  // namespace specq

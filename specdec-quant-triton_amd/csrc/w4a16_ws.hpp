@@ -57,7 +57,7 @@ struct W4WsCfg {
 // compiler's wait-count pass can then tell that reads of one slot do not depend on the DMA
 // still filling another.  Also inlined into the plan-mode launch that holds several tilings
 // (w4a16_plan.hpp), which passes slots sized for its largest tiling.
-template <int MT, int RW, int S, int NSLOT, int NSW, int LAYOUT, class SlotPtr>
+template <int MT, int RW, int S, int NSLOT, int NSW, int LAYOUT, bool KEEP, class SlotPtr>
 __device__ __forceinline__ void w4a16_ws_body(W4A16Params p, SlotPtr slot_ptr) {
   using C = W4WsCfg<MT, RW, S, NSLOT, NSW, LAYOUT>;
   static_assert(C::OK, "unsupported W4A16 weight-stream tile");
@@ -116,7 +116,7 @@ __device__ __forceinline__ void w4a16_ws_body(W4A16Params p, SlotPtr slot_ptr) {
     }
   };
 
-  W4Weights<RW, LAYOUT> wt;
+  W4Weights<RW, LAYOUT, KEEP> wt;
   wt.init(p, n0);
   auto w_issue = [&](int c, int j, v4i (&wq)[RW], uint32_t (&sv)[RW][NSC]) {
     const int q = c * S + j;
@@ -260,18 +260,29 @@ __device__ __forceinline__ void w4a16_ws_body(W4A16Params p, SlotPtr slot_ptr) {
 
 constexpr int kW4WsThreads = 512;  // the split-K finish above is instantiated for 512 threads
 
-template <int MT, int RW, int S, int NSLOT, int NSW, int LAYOUT>
-__global__ __launch_bounds__(kW4WsThreads) void w4a16_ws_kernel(W4A16Params p) {
+template <int MT, int RW, int S, int NSLOT, int NSW, int LAYOUT, bool KEEP>
+__device__ __forceinline__ void w4a16_ws_entry(const W4A16Params& p) {
   constexpr int SLOT = W4WsCfg<MT, RW, S, NSLOT, NSW, LAYOUT>::SLOT;
   __shared__ __attribute__((aligned(16))) uint8_t lds_s0[2][SLOT], lds_s1[2][SLOT];
   __shared__ __attribute__((aligned(16))) uint8_t lds_s2[2][NSLOT > 2 ? SLOT : 16], lds_s3[2][NSLOT > 3 ? SLOT : 16];
-  w4a16_ws_body<MT, RW, S, NSLOT, NSW, LAYOUT>(p, [&](auto ic, int h) -> uint8_t* {
+  w4a16_ws_body<MT, RW, S, NSLOT, NSW, LAYOUT, KEEP>(p, [&](auto ic, int h) -> uint8_t* {
     constexpr int i = decltype(ic)::value;
     if constexpr (i == 0) return lds_s0[h];
     else if constexpr (i == 1) return lds_s1[h];
     else if constexpr (i == 2) return lds_s2[h];
     else return lds_s3[h];
   });
+}
+
+template <int MT, int RW, int S, int NSLOT, int NSW, int LAYOUT>
+__global__ __launch_bounds__(kW4WsThreads) void w4a16_ws_kernel(W4A16Params p) {
+  w4a16_ws_entry<MT, RW, S, NSLOT, NSW, LAYOUT, false>(p);
+}
+// Eager launches of several M-chunks: the chunks of a channel tile share an XCD, and its L2 serves
+// the weight to all but the first.
+template <int MT, int RW, int S, int NSLOT, int NSW, int LAYOUT>
+__global__ __launch_bounds__(kW4WsThreads) void w4a16_chunks_ws_kernel(W4A16Params p) {
+  w4a16_ws_entry<MT, RW, S, NSLOT, NSW, LAYOUT, true>(p);
 }
 
 }  // namespace specq

@@ -4,28 +4,28 @@
 
 namespace specq {
 
-const void* w4a16_ws_fn_l2(int mt, int rw) {
+const void* w4a16_ws_fn_l2(int mt, int rw, bool keep) {
   switch (mt * 4 + rw) {
-    case 5: return w4a16_ws_pick<1, 1, 2>();
-    case 6: return w4a16_ws_pick<1, 2, 2>();
-    case 9: return w4a16_ws_pick<2, 1, 2>();
-    case 10: return w4a16_ws_pick<2, 2, 2>();
-    case 13: return w4a16_ws_pick<3, 1, 2>();
-    case 14: return w4a16_ws_pick<3, 2, 2>();
-    case 17: return w4a16_ws_pick<4, 1, 2>();
-    case 18: return w4a16_ws_pick<4, 2, 2>();
-    case 21: return w4a16_ws_pick<5, 1, 2>();
-    case 22: return w4a16_ws_pick<5, 2, 2>();
-    case 25: return w4a16_ws_pick<6, 1, 2>();
-    case 26: return w4a16_ws_pick<6, 2, 2>();
-    case 29: return w4a16_ws_pick<7, 1, 2>();
-    case 30: return w4a16_ws_pick<7, 2, 2>();
-    case 33: return w4a16_ws_pick<8, 1, 2>();
-    case 34: return w4a16_ws_pick<8, 2, 2>();
-    case 37: return w4a16_ws_pick<9, 1, 2>();
-    case 38: return w4a16_ws_pick<9, 2, 2>();
-    case 41: return w4a16_ws_pick<10, 1, 2>();
-    case 42: return w4a16_ws_pick<10, 2, 2>();
+    case 5: return w4a16_ws_pick<1, 1, 2>(keep);
+    case 6: return w4a16_ws_pick<1, 2, 2>(keep);
+    case 9: return w4a16_ws_pick<2, 1, 2>(keep);
+    case 10: return w4a16_ws_pick<2, 2, 2>(keep);
+    case 13: return w4a16_ws_pick<3, 1, 2>(keep);
+    case 14: return w4a16_ws_pick<3, 2, 2>(keep);
+    case 17: return w4a16_ws_pick<4, 1, 2>(keep);
+    case 18: return w4a16_ws_pick<4, 2, 2>(keep);
+    case 21: return w4a16_ws_pick<5, 1, 2>(keep);
+    case 22: return w4a16_ws_pick<5, 2, 2>(keep);
+    case 25: return w4a16_ws_pick<6, 1, 2>(keep);
+    case 26: return w4a16_ws_pick<6, 2, 2>(keep);
+    case 29: return w4a16_ws_pick<7, 1, 2>(keep);
+    case 30: return w4a16_ws_pick<7, 2, 2>(keep);
+    case 33: return w4a16_ws_pick<8, 1, 2>(keep);
+    case 34: return w4a16_ws_pick<8, 2, 2>(keep);
+    case 37: return w4a16_ws_pick<9, 1, 2>(keep);
+    case 38: return w4a16_ws_pick<9, 2, 2>(keep);
+    case 41: return w4a16_ws_pick<10, 1, 2>(keep);
+    case 42: return w4a16_ws_pick<10, 2, 2>(keep);
     default: return nullptr;
   }
 }

@@ -85,3 +85,17 @@ def test_many_rows_over_wide_strides():
     torch.cuda.synchronize()
     assert "deep_kernel" in ck.name, ck.name
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("block_m", [80, 96, 112, 128, 144, 160])
+@pytest.mark.parametrize("layout, rows", [("packed", 1), ("packed", 161), ("u8", 17), ("i32", 40)])
+def test_several_chunks_of_the_streaming_kernel(block_m, layout, rows):
+    """Two and three M-chunks, the last ragged: the bits of 64-row tiles, whose weight loads are the other kind."""
+    M, N, Kd = block_m + rows, 1030, 1280
+    note(f"w4a16 chunks {layout} M={M} BLOCK_M={block_m}")
+    a, wp, sc, _ = operands(layout, M, N, Kd, 128, seed=block_m)
+    out, ck = K.w4a16_matmul(a, wp, sc, BLOCK_M=block_m)
+    ref, ck64 = K.w4a16_matmul(a, wp, sc, BLOCK_M=64)
+    torch.cuda.synchronize()
+    assert "chunks_ws_kernel" in ck.name and "w4a16_ws_kernel" in ck64.name, (ck.name, ck64.name)
+    assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), ck.name
