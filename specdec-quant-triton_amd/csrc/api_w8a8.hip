@@ -150,6 +150,7 @@ struct W8A8Cfg {
   int mt, rw, nw, vec, splits, k_range, n_tiles, m_chunks;
   int bn;         // channels per workgroup
   int deep;       // kDeep: the many-row tile (DeepTile)
+  bool keep = false;  // kWs: weights stay in L2 for the other M-chunks
   int bnsel;      // RK/WS channel-width variant (0..3 for 16/32/64/128)
   size_t lds, ws_partials, ws_counters;
   const void* fn;
@@ -176,20 +177,20 @@ const void* legacy_fn(int mt, int rw, int vec) {
   return nullptr;
 }
 
-const void* ws_fn(int bnsel, int layout, int mt) {
+const void* ws_fn(int bnsel, int layout, int mt, bool keep) {
   switch (bnsel * 3 + layout) {
-    case 0: return w8a8_ws_fn_n16_l0(mt);
-    case 1: return w8a8_ws_fn_n16_l1(mt);
-    case 2: return w8a8_ws_fn_n16_l2(mt);
-    case 3: return w8a8_ws_fn_n32_l0(mt);
-    case 4: return w8a8_ws_fn_n32_l1(mt);
-    case 5: return w8a8_ws_fn_n32_l2(mt);
-    case 6: return w8a8_ws_fn_n64_l0(mt);
-    case 7: return w8a8_ws_fn_n64_l1(mt);
-    case 8: return w8a8_ws_fn_n64_l2(mt);
-    case 9: return w8a8_ws_fn_n128_l0(mt);
-    case 10: return w8a8_ws_fn_n128_l1(mt);
-    case 11: return w8a8_ws_fn_n128_l2(mt);
+    case 0: return w8a8_ws_fn_n16_l0(mt, keep);
+    case 1: return w8a8_ws_fn_n16_l1(mt, keep);
+    case 2: return w8a8_ws_fn_n16_l2(mt, keep);
+    case 3: return w8a8_ws_fn_n32_l0(mt, keep);
+    case 4: return w8a8_ws_fn_n32_l1(mt, keep);
+    case 5: return w8a8_ws_fn_n32_l2(mt, keep);
+    case 6: return w8a8_ws_fn_n64_l0(mt, keep);
+    case 7: return w8a8_ws_fn_n64_l1(mt, keep);
+    case 8: return w8a8_ws_fn_n64_l2(mt, keep);
+    case 9: return w8a8_ws_fn_n128_l0(mt, keep);
+    case 10: return w8a8_ws_fn_n128_l1(mt, keep);
+    case 11: return w8a8_ws_fn_n128_l2(mt, keep);
   }
   return nullptr;
 }
@@ -449,7 +450,10 @@ int w8a8_config(int layout, int m_grid, int N, int K, int block_m, int block_n, 
       }
       fn = w8a8_rk_fn(bnsel, layout);
     } else {
-      fn = ws_fn(bnsel, layout, mt);
+      // Weights that several M-chunks read stay in L2; with one chunk they are read once and do not
+      // (N = 28672, K = 4096, M = 72: 22.4 us, and 23.7 kept).
+      cfg->keep = !plan_mode && m_grid > mt * 16 && w8a8_ws_keeps(mt, bnsel, layout);
+      fn = ws_fn(bnsel, layout, mt, cfg->keep);
     }
   }
   if (family == kLegacy) {
@@ -820,7 +824,7 @@ int w8a8_attrs(int layout, int m_grid, int N, int K, int block_m, int block_n, i
     snprintf(out->name, sizeof(out->name), "specq::w8a8_rk_kernel<1, %d, %d, 4, %d>", rw, kw, cfg.layout);
   } else if (cfg.family == kWs) {
     const int nslot = w8a8_ws_nslot(cfg.mt, kw);
-    snprintf(out->name, sizeof(out->name), "specq::w8a8_ws_kernel<%d, %d, %d, %d, %d, 4, %d>", cfg.mt, rw, kw, s,
+    snprintf(out->name, sizeof(out->name), "specq::w8a8_%sws_kernel<%d, %d, %d, %d, %d, 4, %d>", cfg.keep ? "chunks_" : "", cfg.mt, rw, kw, s,
              nslot, cfg.layout);
   } else {
     snprintf(out->name, sizeof(out->name), "specq::w8a8_kernel<%d, %d, %d>", cfg.mt, cfg.rw, cfg.vec);

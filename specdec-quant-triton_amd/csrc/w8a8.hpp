@@ -109,12 +109,13 @@ template <> struct W8A8WFragT<2> { using type = v2i; };
 template <int WL> using W8A8WFrag = typename W8A8WFragT<WL>::type;
 template <int WL> struct W8A8WFragBytes { static constexpr uint32_t value = WL == 2 ? 512u : 1024u; };
 
-template <int WL>
+// Non-temporal; KEEP: the line stays in L2 for the other workgroups that read it.
+template <int WL, bool KEEP = false>
 __device__ __forceinline__ W8A8WFrag<WL> w8a8_wload(rsrc_t rs, uint32_t off) {
   if constexpr (WL == 2) {
-    return __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, 2));
+    return __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rs, off, 0, KEEP ? 0 : 2));
   } else {
-    return __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 2);
+    return __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, KEEP ? 0 : 2);
   }
 }
 

@@ -65,7 +65,7 @@ __device__ __forceinline__ void w8a8_plan_path(const W8A8Params& p, SlotPtr slot
     using P = W8A8WsPick<MT, SEL>;
     static_assert(P::Cfg::SLOT <= kW8A8PlanSlotA[V] && (P::NSLOT <= 2 || P::Cfg::SLOT <= kW8A8PlanSlotB[V]),
                   "menu tiling fits the shared slots");
-    w8a8_ws_body<MT, B::RW, B::KW, B::S, P::NSLOT, 4, WL>(p, slots);
+    w8a8_ws_body<MT, B::RW, B::KW, B::S, P::NSLOT, 4, WL, false>(p, slots);
   }
 }
 

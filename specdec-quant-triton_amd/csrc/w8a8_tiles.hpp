@@ -35,10 +35,20 @@ struct W8A8WsPick {
   using Cfg = W8A8WsCfg<MT, B::RW, B::KW, B::S, NSLOT, 4>;
 };
 
+// Tiles of packed INT8 weights that automatic tiles run in several M-chunks (48 rows, 64 channels and
+// up) also come with weight loads that stay in L2 (w8a8_chunks_ws_kernel), for launches that have them
+// (non-temporal -> kept, us: N = 10000, K = 3072, M = 128 14.5 -> 12.8; N = 4096, K = 14336, M = 288 38.5 ->
+// 36.4, 517 53.2 -> 51.7; N = 3072, K = 8192, M = 256 20.9 -> 20.0).  INT4 fragments, half as long, do
+// not: N = 5120, K = 13824, M = 288 38.6 -> 40.3.
+constexpr bool w8a8_ws_keeps(int mt, int bnsel, int layout) { return mt >= 3 && bnsel >= 2 && layout == 1; }
+
 template <int MT, int BNSEL, int WL>
-const void* w8a8_ws_pick() {
+const void* w8a8_ws_pick(bool keep) {
   using P = W8A8WsPick<MT, BNSEL>;
   using B = W8A8BnSel<BNSEL>;
+  if constexpr (w8a8_ws_keeps(MT, BNSEL, WL)) {
+    if (keep) return reinterpret_cast<const void*>(&w8a8_chunks_ws_kernel<MT, B::RW, B::KW, B::S, P::NSLOT, 4, WL>);
+  }
   return reinterpret_cast<const void*>(&w8a8_ws_kernel<MT, B::RW, B::KW, B::S, P::NSLOT, 4, WL>);
 }
 
@@ -49,18 +59,18 @@ const void* w8a8_rk_pick() {
 }
 
 // Defined in the instantiation units.
-const void* w8a8_ws_fn_n16_l0(int mt);
-const void* w8a8_ws_fn_n16_l1(int mt);
-const void* w8a8_ws_fn_n32_l0(int mt);
-const void* w8a8_ws_fn_n32_l1(int mt);
-const void* w8a8_ws_fn_n64_l0(int mt);
-const void* w8a8_ws_fn_n64_l1(int mt);
-const void* w8a8_ws_fn_n128_l0(int mt);
-const void* w8a8_ws_fn_n128_l1(int mt);
-const void* w8a8_ws_fn_n16_l2(int mt);
-const void* w8a8_ws_fn_n32_l2(int mt);
-const void* w8a8_ws_fn_n64_l2(int mt);
-const void* w8a8_ws_fn_n128_l2(int mt);
+const void* w8a8_ws_fn_n16_l0(int mt, bool keep);
+const void* w8a8_ws_fn_n16_l1(int mt, bool keep);
+const void* w8a8_ws_fn_n32_l0(int mt, bool keep);
+const void* w8a8_ws_fn_n32_l1(int mt, bool keep);
+const void* w8a8_ws_fn_n64_l0(int mt, bool keep);
+const void* w8a8_ws_fn_n64_l1(int mt, bool keep);
+const void* w8a8_ws_fn_n128_l0(int mt, bool keep);
+const void* w8a8_ws_fn_n128_l1(int mt, bool keep);
+const void* w8a8_ws_fn_n16_l2(int mt, bool keep);
+const void* w8a8_ws_fn_n32_l2(int mt, bool keep);
+const void* w8a8_ws_fn_n64_l2(int mt, bool keep);
+const void* w8a8_ws_fn_n128_l2(int mt, bool keep);
 const void* w8a8_rk_fn(int bnsel, int layout);
 
 }  // namespace specq

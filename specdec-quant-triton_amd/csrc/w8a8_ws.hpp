@@ -58,7 +58,7 @@ struct W8A8WsCfg {
 // variables: the compiler's wait-count pass can then tell that reads of one slot do not
 // depend on the DMA still filling another.  Also inlined into the plan-mode launch that holds
 // several tilings (w8a8_plan.hpp), which passes slots sized for its largest tiling.
-template <int MT, int RW, int KW, int S, int NSLOT, int NW, int WL, class SlotPtr>
+template <int MT, int RW, int KW, int S, int NSLOT, int NW, int WL, bool KEEP, class SlotPtr>
 __device__ __forceinline__ void w8a8_ws_body(W8A8Params p, SlotPtr slot_ptr) {
   using C = W8A8WsCfg<MT, RW, KW, S, NSLOT, NW>;
   static_assert(C::OK, "unsupported W8A8 weight-stream tile");
@@ -152,7 +152,7 @@ __device__ __forceinline__ void w8a8_ws_body(W8A8Params p, SlotPtr slot_ptr) {
 #pragma unroll
     for (int t = 0; t < RW; ++t) {
       const uint32_t off = oob_unless(live & (wrow[t] != kOOB), wrow[t] + (uint32_t)step * sstride);
-      slot[t] = w8a8_wload<WL>(wsrc, off);
+      slot[t] = w8a8_wload<WL, KEEP>(wsrc, off);
     }
   };
 
@@ -332,13 +332,13 @@ __device__ __forceinline__ void w8a8_ws_body(W8A8Params p, SlotPtr slot_ptr) {
   tl_mark_drained(p.tl, p.tl_cap, 4);  // diagnostics build: hand-off (and, if last, the sum) done
 }
 
-template <int MT, int RW, int KW, int S, int NSLOT, int NW, int WL>
-__global__ __launch_bounds__(NW * 64) void w8a8_ws_kernel(W8A8Params p) {
+template <int MT, int RW, int KW, int S, int NSLOT, int NW, int WL, bool KEEP>
+__device__ __forceinline__ void w8a8_ws_entry(const W8A8Params& p) {
   constexpr int SLOT = W8A8WsCfg<MT, RW, KW, S, NSLOT, NW>::SLOT;
   __shared__ __attribute__((aligned(16))) uint8_t lds_s0[SLOT], lds_s1[SLOT];
   __shared__ __attribute__((aligned(16))) uint8_t lds_s2[NSLOT > 2 ? SLOT : 16], lds_s3[NSLOT > 3 ? SLOT : 16];
   __shared__ __attribute__((aligned(16))) uint8_t lds_s4[NSLOT > 4 ? SLOT : 16], lds_s5[NSLOT > 5 ? SLOT : 16];
-  w8a8_ws_body<MT, RW, KW, S, NSLOT, NW, WL>(p, [&](auto ic) -> uint8_t* {
+  w8a8_ws_body<MT, RW, KW, S, NSLOT, NW, WL, KEEP>(p, [&](auto ic) -> uint8_t* {
     constexpr int i = decltype(ic)::value;
     if constexpr (i == 0) return lds_s0;
     else if constexpr (i == 1) return lds_s1;
@@ -347,6 +347,17 @@ __global__ __launch_bounds__(NW * 64) void w8a8_ws_kernel(W8A8Params p) {
     else if constexpr (i == 4) return lds_s4;
     else return lds_s5;
   });
+}
+
+template <int MT, int RW, int KW, int S, int NSLOT, int NW, int WL>
+__global__ __launch_bounds__(NW * 64) void w8a8_ws_kernel(W8A8Params p) {
+  w8a8_ws_entry<MT, RW, KW, S, NSLOT, NW, WL, false>(p);
+}
+// Eager launches of several M-chunks: the chunks of a channel tile share an XCD, and its L2 serves
+// the weight to all but the first.
+template <int MT, int RW, int KW, int S, int NSLOT, int NW, int WL>
+__global__ __launch_bounds__(NW * 64) void w8a8_chunks_ws_kernel(W8A8Params p) {
+  w8a8_ws_entry<MT, RW, KW, S, NSLOT, NW, WL, true>(p);
 }
 
 }  // namespace specq

@@ -4,26 +4,26 @@
 
 namespace specq {
 
-const void* w8a8_ws_fn_n32_l1(int mt) {
+const void* w8a8_ws_fn_n32_l1(int mt, bool keep) {
   switch (mt) {
-    case 2: return w8a8_ws_pick<2, 1, 1>();
-    case 3: return w8a8_ws_pick<3, 1, 1>();
-    case 4: return w8a8_ws_pick<4, 1, 1>();
-    case 5: return w8a8_ws_pick<5, 1, 1>();
-    case 6: return w8a8_ws_pick<6, 1, 1>();
-    case 7: return w8a8_ws_pick<7, 1, 1>();
-    case 8: return w8a8_ws_pick<8, 1, 1>();
-    case 9: return w8a8_ws_pick<9, 1, 1>();
-    case 10: return w8a8_ws_pick<10, 1, 1>();
-    case 11: return w8a8_ws_pick<11, 1, 1>();
-    case 12: return w8a8_ws_pick<12, 1, 1>();
-    case 13: return w8a8_ws_pick<13, 1, 1>();
-    case 14: return w8a8_ws_pick<14, 1, 1>();
-    case 15: return w8a8_ws_pick<15, 1, 1>();
-    case 16: return w8a8_ws_pick<16, 1, 1>();
-    case 17: return w8a8_ws_pick<17, 1, 1>();
-    case 18: return w8a8_ws_pick<18, 1, 1>();
-    case 19: return w8a8_ws_pick<19, 1, 1>();
+    case 2: return w8a8_ws_pick<2, 1, 1>(keep);
+    case 3: return w8a8_ws_pick<3, 1, 1>(keep);
+    case 4: return w8a8_ws_pick<4, 1, 1>(keep);
+    case 5: return w8a8_ws_pick<5, 1, 1>(keep);
+    case 6: return w8a8_ws_pick<6, 1, 1>(keep);
+    case 7: return w8a8_ws_pick<7, 1, 1>(keep);
+    case 8: return w8a8_ws_pick<8, 1, 1>(keep);
+    case 9: return w8a8_ws_pick<9, 1, 1>(keep);
+    case 10: return w8a8_ws_pick<10, 1, 1>(keep);
+    case 11: return w8a8_ws_pick<11, 1, 1>(keep);
+    case 12: return w8a8_ws_pick<12, 1, 1>(keep);
+    case 13: return w8a8_ws_pick<13, 1, 1>(keep);
+    case 14: return w8a8_ws_pick<14, 1, 1>(keep);
+    case 15: return w8a8_ws_pick<15, 1, 1>(keep);
+    case 16: return w8a8_ws_pick<16, 1, 1>(keep);
+    case 17: return w8a8_ws_pick<17, 1, 1>(keep);
+    case 18: return w8a8_ws_pick<18, 1, 1>(keep);
+    case 19: return w8a8_ws_pick<19, 1, 1>(keep);
     default: return nullptr;
   }
 }

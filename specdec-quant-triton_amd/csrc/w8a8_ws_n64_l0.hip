@@ -4,26 +4,26 @@
 
 namespace specq {
 
-const void* w8a8_ws_fn_n64_l0(int mt) {
+const void* w8a8_ws_fn_n64_l0(int mt, bool keep) {
   switch (mt) {
-    case 2: return w8a8_ws_pick<2, 2, 0>();
-    case 3: return w8a8_ws_pick<3, 2, 0>();
-    case 4: return w8a8_ws_pick<4, 2, 0>();
-    case 5: return w8a8_ws_pick<5, 2, 0>();
-    case 6: return w8a8_ws_pick<6, 2, 0>();
-    case 7: return w8a8_ws_pick<7, 2, 0>();
-    case 8: return w8a8_ws_pick<8, 2, 0>();
-    case 9: return w8a8_ws_pick<9, 2, 0>();
-    case 10: return w8a8_ws_pick<10, 2, 0>();
-    case 11: return w8a8_ws_pick<11, 2, 0>();
-    case 12: return w8a8_ws_pick<12, 2, 0>();
-    case 13: return w8a8_ws_pick<13, 2, 0>();
-    case 14: return w8a8_ws_pick<14, 2, 0>();
-    case 15: return w8a8_ws_pick<15, 2, 0>();
-    case 16: return w8a8_ws_pick<16, 2, 0>();
-    case 17: return w8a8_ws_pick<17, 2, 0>();
-    case 18: return w8a8_ws_pick<18, 2, 0>();
-    case 19: return w8a8_ws_pick<19, 2, 0>();
+    case 2: return w8a8_ws_pick<2, 2, 0>(keep);
+    case 3: return w8a8_ws_pick<3, 2, 0>(keep);
+    case 4: return w8a8_ws_pick<4, 2, 0>(keep);
+    case 5: return w8a8_ws_pick<5, 2, 0>(keep);
+    case 6: return w8a8_ws_pick<6, 2, 0>(keep);
+    case 7: return w8a8_ws_pick<7, 2, 0>(keep);
+    case 8: return w8a8_ws_pick<8, 2, 0>(keep);
+    case 9: return w8a8_ws_pick<9, 2, 0>(keep);
+    case 10: return w8a8_ws_pick<10, 2, 0>(keep);
+    case 11: return w8a8_ws_pick<11, 2, 0>(keep);
+    case 12: return w8a8_ws_pick<12, 2, 0>(keep);
+    case 13: return w8a8_ws_pick<13, 2, 0>(keep);
+    case 14: return w8a8_ws_pick<14, 2, 0>(keep);
+    case 15: return w8a8_ws_pick<15, 2, 0>(keep);
+    case 16: return w8a8_ws_pick<16, 2, 0>(keep);
+    case 17: return w8a8_ws_pick<17, 2, 0>(keep);
+    case 18: return w8a8_ws_pick<18, 2, 0>(keep);
+    case 19: return w8a8_ws_pick<19, 2, 0>(keep);
     default: return nullptr;
   }
 }

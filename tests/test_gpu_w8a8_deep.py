@@ -104,3 +104,18 @@ def test_many_rows_over_wide_strides():
     torch.cuda.synchronize()
     assert "deep_kernel<2, 4, 3, 1>" in ck.name, ck.name
     assert torch.equal(out.view(torch.int16), formula(a, sa, w, sw).view(torch.int16)), ck.name
+
+
+@pytest.mark.parametrize("block_m", [48, 64, 128, 208, 304])
+@pytest.mark.parametrize("block_n, split_k", [(64, 1), (64, 3), (128, 1), (128, 4)])
+def test_several_chunks_of_the_streaming_kernel(block_m, block_n, split_k):
+    """Two and three M-chunks, the last ragged, whose weight loads stay in L2; one chunk keeps the other kind."""
+    N, Kd = 1030, 1296
+    note(f"w8a8 chunks BLOCK_M={block_m} BLOCK_N={block_n} split_k={split_k}")
+    a, sa, wp, sw, w = operands("w8a8", 2 * block_m + 1, N, Kd, seed=block_m)
+    kw = dict(BLOCK_M=block_m, BLOCK_N=block_n, split_k=split_k)
+    for M, name in ((block_m, "w8a8_ws_kernel"), (block_m + 17, "chunks_ws_kernel"), (2 * block_m + 1, "chunks_ws_kernel")):
+        out, ck = K.w8a8_matmul(a[:M], sa[:M], wp, sw, **kw)
+        torch.cuda.synchronize()
+        assert name in ck.name, (M, ck.name)
+        assert torch.equal(out.view(torch.int16), formula(a[:M], sa[:M], w, sw).view(torch.int16)), (M, ck.name)
