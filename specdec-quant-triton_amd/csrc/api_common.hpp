@@ -26,6 +26,9 @@ inline int fail(int code, const char* what) {
     }                                  \
   } while (0)
 
+// Whether a many-row tile's rows, ld bytes apart and len bytes long, reach past the 4 GiB of a buffer resource.
+inline bool deep_wide(int rows, int64_t ld, int64_t len) { return (rows - 1) * ld + len > 0xFFFFFFFFll; }
+
 // Flag in the `variant` of a GEMM resource query: the call ran with a plan (tile rules differ).
 constexpr int kAttrsPlan = 16;
 // ... or the tiles are for an explicit request (W8A8: no many-row tile, which none names).

@@ -472,6 +472,7 @@ extern "C" int specq_w4a16(const void* a, int64_t lda, const void* wq, int64_t l
     for (int e = 0; e < kW4PlanRows; ++e) pp.t[e] = cfg.plan_t[e];
     return launch(cfg.fn, cfg.grid, kW4WsThreads, 0, (hipStream_t)stream, &pp);
   }
+  if (cfg.family == kW4Deep && deep_wide(std::min(cfg.mt * 16, M), lda * 2, K * (int64_t)2)) cfg.fn = w4a16_deep_fn(wq_layout, true);
   return launch(cfg.fn, cfg.grid, cfg.family == kW4Rk ? 256 : kW4WsThreads, 0, (hipStream_t)stream, &p);
 }
 
@@ -574,6 +575,7 @@ extern "C" int specq_w4a16_grouped(const void* a, int64_t lda, int n_members, co
     p.grp_ntiles16[g - 1] = on ? ceil_div(N[g], 16) : 0;
     p.grp_vec_store[g - 1] = on ? vec_ok(g) : 0;
   }
+  if (cfg.family == kW4Deep && deep_wide(std::min(cfg.mt * 16, M), lda * 2, K * (int64_t)2)) cfg.fn = w4a16_deep_fn(wq_layout, true);
   return launch(cfg.fn, cfg.grid, cfg.family == kW4Rk ? 256 : kW4WsThreads, 0, (hipStream_t)stream, &p);
 }
 

@@ -742,7 +742,10 @@ int run_w8a8(int layout, const int8_t* a, int64_t lda, const W8A8Group& grp, con
     }
   }
   int grid = cfg.family == kPlan ? cfg.plan_grid : chunked_grid(cfg.n_tiles * cfg.splits, cfg.m_chunks);
-  if (cfg.family == kDeep) grid = w8a8_deep_grid(cfg, &p.whole);
+  if (cfg.family == kDeep) {
+    grid = w8a8_deep_grid(cfg, &p.whole);
+    if (deep_wide(std::min(kDeepRows[cfg.deep], M), lda, K)) cfg.fn = w8a8_deep_fn(cfg.deep, layout, true);
+  }
   if (static_scratch && need) {
     int n_ctr = cfg.family == kPlan ? cfg.n_counters : cfg.m_chunks * cfg.n_tiles;
     int32_t* ctr = p.counters;

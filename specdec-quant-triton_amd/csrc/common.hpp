@@ -340,12 +340,24 @@ __device__ __forceinline__ void deep_dma(v4i rs, uint32_t voff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rs), "s"(lds)
                : "memory", "m0");
 }
-// Raw buffer resource over n bytes from base (none when n <= 0, at most 2^32 - 1: offsets are unsigned).
-__device__ __forceinline__ v4i deep_rsrc(const void* base, int64_t n) {
+// Bytes of a buffer that holds n, as a resource counts them: none when n <= 0, at most 2^32 - 1.
+__device__ __forceinline__ uint32_t deep_extent(int64_t n) {
+  return n < 0 ? 0u : (n > 0xFFFFFFFFll ? 0xFFFFFFFFu : (uint32_t)n);
+}
+// Raw buffer resource over n bytes from base (offsets are unsigned).
+__device__ __forceinline__ v4i deep_rsrc(const void* base, uint32_t n) {
   const uint64_t a = (uint64_t)(uintptr_t)base;
-  const int64_t m = n < 0 ? 0 : (n > 0xFFFFFFFFll ? 0xFFFFFFFFll : n);
-  return v4i{uniform((int)(uint32_t)a), uniform((int)((uint32_t)(a >> 32) & 0xFFFFu)), uniform((int)(uint32_t)m),
-             kRsrcWord3};
+  return v4i{uniform((int)(uint32_t)a), uniform((int)((uint32_t)(a >> 32) & 0xFFFFu)), uniform((int)n), kRsrcWord3};
+}
+
+// The resource of an activation DMA of R rows from row `row` of a tile's m_rows (ld bytes apart, from a;
+// the k-th of len bytes on).  Worked out where it is used: held over the loop, the resources of all of a
+// wave's DMAs take more scalar registers than there are.
+template <int R>
+__device__ __forceinline__ v4i deep_rows_rsrc(const void* a, int row, int m_rows, int64_t ld, int64_t k, int64_t len) {
+  asm volatile("" : "+s"(row));
+  const int64_t n = (min(R, m_rows - row) - 1) * ld + len - k;  // up to the end of the last row
+  return deep_rsrc(reinterpret_cast<const uint8_t*>(a) + row * ld + k, row < m_rows ? deep_extent(n) : 0u);
 }
 
 __device__ __forceinline__ void wait_all_memory() {

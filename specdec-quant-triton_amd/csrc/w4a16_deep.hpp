@@ -35,8 +35,8 @@
 
 namespace specq {
 
-template <int LAYOUT>
-__global__ __launch_bounds__(512) void w4a16_deep_kernel(W4A16Params p) {
+template <int LAYOUT, bool WIDE>
+__device__ __forceinline__ void w4a16_deep_entry(W4A16Params p) {
   constexpr int FM = 4, FN = 4, BM = 128, BN = 128;
   constexpr int NSC = W4Nsc<LAYOUT>::value;
   constexpr int SLOT = BM * 256;           // activation bytes of a block
@@ -68,7 +68,9 @@ __global__ __launch_bounds__(512) void w4a16_deep_kernel(W4A16Params p) {
   auto block = [&](const Cursor& c) { return c.first + 2 * c.q + h; };
 
   // ---- Activation DMA i of a block: rows 4 (w A_L + i) .. + 3, lane l piece (l % 16) ^ (row % 16)
-  // of the row's 256 bytes (layout 0: 128 bytes at K and 128 at K + K/2).
+  // of the row's 256 bytes (layout 0: 128 bytes at K and 128 at K + K/2).  WIDE: a tile's rows may span
+  // more than the 4 GiB of a resource, so each DMA has one of its own from its first row on and a lane's
+  // 32-bit offset covers that DMA's four rows only (row strides up to 1 GiB).
   const int m_rows = min(BM, M - m0);
   const uint8_t* a0 = reinterpret_cast<const uint8_t*>(p.A + (int64_t)m0 * p.lda);
   const int64_t a_bytes = ((int64_t)(m_rows - 1) * p.lda + p.K) * 2;
@@ -77,14 +79,18 @@ __global__ __launch_bounds__(512) void w4a16_deep_kernel(W4A16Params p) {
 #pragma unroll
   for (int i = 0; i < A_L; ++i) {
     const int row = 4 * (w * A_L + i) + g, c = r ^ (row & 15);
-    a_off[i] = (uint32_t)row * (uint32_t)p.lda * 2 + (LAYOUT == 0 ? (c < 8 ? 16 * c : p.K + 16 * (c - 8)) : 16 * c);
+    a_off[i] = (uint32_t)(WIDE ? g : row) * (uint32_t)p.lda * 2 +
+               (LAYOUT == 0 ? (c < 8 ? 16 * c : p.K + 16 * (c - 8)) : 16 * c);
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds + (uint32_t)(h * 2 * SLOT + w * A_L * 1024);
   auto dma = [&](const Cursor& c, int slot) __attribute__((always_inline)) {
     const int64_t k = (int64_t)block(c) * kBlockBytes;
-    const v4i rs = deep_rsrc(a0 + k, live(c) ? a_bytes - k : 0);
 #pragma unroll
-    for (int i = 0; i < A_L; ++i) deep_dma(rs, a_off[i], lds0 + (uint32_t)(slot * SLOT + i * 1024));
+    for (int i = 0; i < A_L; ++i) {
+      const v4i rs = WIDE ? deep_rows_rsrc<4>(a0, 4 * (w * A_L + i), live(c) ? m_rows : 0, 2 * p.lda, k, 2 * (int64_t)p.K)
+                          : deep_rsrc(a0 + k, deep_extent(live(c) ? a_bytes - k : 0));
+      deep_dma(rs, a_off[i], lds0 + (uint32_t)(slot * SLOT + i * 1024));
+    }
   };
   const uint8_t* a_rd = lds + h * 2 * SLOT + (wm * FM * 16 + r) * 256;
   int pc[4];  // LDS position of the lane's piece of MFMA step u
@@ -210,7 +216,12 @@ __global__ __launch_bounds__(512) void w4a16_deep_kernel(W4A16Params p) {
   tl_mark_drained(p.tl, p.tl_cap, 4);  // ... and completed
 }
 
-// Defined in the instantiation unit.
-const void* w4a16_deep_fn(int layout);
+template <int LAYOUT>
+__global__ __launch_bounds__(512) void w4a16_deep_kernel(W4A16Params p) { w4a16_deep_entry<LAYOUT, false>(p); }
+template <int LAYOUT>
+__global__ __launch_bounds__(512) void w4a16_deep_wide_kernel(W4A16Params p) { w4a16_deep_entry<LAYOUT, true>(p); }
+
+// Defined in the instantiation unit (`wide`: the kernel for rows that span more than 4 GiB within a tile).
+const void* w4a16_deep_fn(int layout, bool wide = false);
 
 }  // namespace specq

@@ -4,16 +4,28 @@
 
 namespace specq {
 
-const void* w8a8_deep_fn(int tile, int layout) {
+namespace {
+
+template <int FM, int FN, int NSL, int WL>
+const void* pick(bool wide) {
+  return wide ? reinterpret_cast<const void*>(&w8a8_deep_wide_kernel<FM, FN, NSL, WL>)
+              : reinterpret_cast<const void*>(&w8a8_deep_kernel<FM, FN, NSL, WL>);
+}
+
+}  // namespace
+
+const void* w8a8_deep_fn(int tile, int layout, bool wide) {
   if (layout == 1) {
     switch (tile) {
-      case kDeep64: return reinterpret_cast<const void*>(&w8a8_deep_kernel<2, 4, 3, 1>);
-      case kDeep128: return reinterpret_cast<const void*>(&w8a8_deep_kernel<4, 4, 4, 1>);
-      case kDeep128Pair: return reinterpret_cast<const void*>(&w8a8_deep_kernel<4, 4, 2, 1>);
-      case kDeepMix: return reinterpret_cast<const void*>(&w8a8_deep_mix_kernel<1>);
+      case kDeep64: return pick<2, 4, 3, 1>(wide);
+      case kDeep128: return pick<4, 4, 4, 1>(wide);
+      case kDeep128Pair: return pick<4, 4, 2, 1>(wide);
+      case kDeepMix:
+        return wide ? reinterpret_cast<const void*>(&w8a8_deep_mix_wide_kernel<1>)
+                    : reinterpret_cast<const void*>(&w8a8_deep_mix_kernel<1>);
     }
   }
-  if (layout == 2 && tile == kDeep128Pair) return reinterpret_cast<const void*>(&w8a8_deep_kernel<4, 4, 2, 2>);
+  if (layout == 2 && tile == kDeep128Pair) return pick<4, 4, 2, 2>(wide);
   return nullptr;
 }
 

@@ -56,8 +56,12 @@ struct W8A8DeepCfg {
   static_assert(NSL >= 2 && LDS <= 160 * 1024 && (NSL - 1) * PER <= 63, "tile");
 };
 
-// One 32 FM x 32 FN tile: rows m0.., channel tile `tile` (launch-wide) of BN channels.
-template <int FM, int FN, int NSL, int WL>
+// One 32 FM x 32 FN tile: rows m0.., channel tile `tile` (launch-wide) of BN channels.  WIDE: a tile's
+// rows may span more than the 4 GiB of a resource, so each activation DMA has one of its own from its
+// first row on and a lane's 32-bit offset covers that DMA's eight rows only (row strides up to 512 MiB).
+// The scalar arithmetic of that between the MFMAs costs 5 % (MLP block of M = 2048, hidden 4096, 14336
+// channels: 366 -> 383 us) and a branch in one kernel its registers, so it is a kernel of its own.
+template <int FM, int FN, int NSL, int WL, bool WIDE>
 __device__ __forceinline__ void w8a8_deep_body(W8A8Params p, uint8_t* lds, int m0, int tile, int M) {
   using C = W8A8DeepCfg<FM, FN, NSL, WL>;
   constexpr int BM = C::BM, BN = C::BN, FB = C::FB;
@@ -66,8 +70,8 @@ __device__ __forceinline__ void w8a8_deep_body(W8A8Params p, uint8_t* lds, int m
   const int wm = w & 1, wn = w >> 1;
   const int nbase = ltile * BN;
 
-  // ---- DMA addresses.  Activation DMA q covers rows 8q .. 8q + 7 of the tile; weight DMA f
-  // covers 1 KB of the chunk's fragments, step-major.  Wave w issues A_L and W_L of them.
+  // ---- DMA addresses.  Activation DMA i of wave w covers rows 8 (w A_L + i) .. + 7 of the tile; weight
+  // DMA f covers 1 KB of the chunk's fragments, step-major.  Wave w issues A_L and W_L of them.
   const int m_rows = min(BM, M - m0);
   const int8_t* a0 = p.A + (int64_t)m0 * p.lda;
   const int64_t a_bytes = (int64_t)(m_rows - 1) * p.lda + p.K;
@@ -79,7 +83,7 @@ __device__ __forceinline__ void w8a8_deep_body(W8A8Params p, uint8_t* lds, int m
 #pragma unroll
   for (int i = 0; i < C::A_L; ++i) {
     const int row = 8 * (w * C::A_L + i) + (lane >> 3);
-    a_off[i] = (uint32_t)row * (uint32_t)p.lda + 16 * ((lane & 7) ^ ((row >> 1) & 7));
+    a_off[i] = (uint32_t)(WIDE ? lane >> 3 : row) * (uint32_t)p.lda + 16 * ((lane & 7) ^ ((row >> 1) & 7));
   }
 #pragma unroll
   for (int i = 0; i < C::W_L; ++i) {
@@ -90,11 +94,13 @@ __device__ __forceinline__ void w8a8_deep_body(W8A8Params p, uint8_t* lds, int m
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)lds;
   auto dma_a = [&](int c, int slot, int i) __attribute__((always_inline)) {
     const int64_t k = (int64_t)c * C::KC;
-    deep_dma(deep_rsrc(a0 + k, a_bytes - k), a_off[i], lds0 + (uint32_t)(slot * C::SLOT + (w * C::A_L + i) * 1024));
+    const v4i rs = WIDE ? deep_rows_rsrc<8>(a0, 8 * (w * C::A_L + i), m_rows, p.lda, k, p.K)
+                        : deep_rsrc(a0 + k, deep_extent(a_bytes - k));
+    deep_dma(rs, a_off[i], lds0 + (uint32_t)(slot * C::SLOT + (w * C::A_L + i) * 1024));
   };
   auto dma_w = [&](int c, int slot, int i) __attribute__((always_inline)) {
     const int64_t o = 2 * step_bytes * c;
-    deep_dma(deep_rsrc(w0 + o, w_bytes - o), w_off[i],
+    deep_dma(deep_rsrc(w0 + o, deep_extent(w_bytes - o)), w_off[i],
              lds0 + (uint32_t)(slot * C::SLOT + C::ASLOT + (w * C::W_L + i) * 1024));
   };
 
@@ -221,19 +227,19 @@ __device__ __forceinline__ int w8a8_deep_rows(const W8A8Params& p) {
   return uniform(p.plan != nullptr ? min(max(p.plan[0], 0), p.m_grid) : p.M);
 }
 
-template <int FM, int FN, int NSL, int WL>
-__global__ __launch_bounds__(256) void w8a8_deep_kernel(W8A8Params p) {
+template <int FM, int FN, int NSL, int WL, bool WIDE>
+__device__ __forceinline__ void w8a8_deep_entry(const W8A8Params& p) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[W8A8DeepCfg<FM, FN, NSL, WL>::LDS];
   tl_mark(p.tl, p.tl_cap, 0);  // diagnostics build: workgroup start
   int mc, tile;
   deep_tile_of(deep_order((int)blockIdx.x, p.m_chunks * p.n_tiles), p.m_chunks, p.n_tiles, mc, tile);
   const int M = w8a8_deep_rows(p), m0 = uniform(mc) * (32 * FM);
-  if (m0 < M) w8a8_deep_body<FM, FN, NSL, WL>(p, lds, m0, uniform(tile), M);
+  if (m0 < M) w8a8_deep_body<FM, FN, NSL, WL, WIDE>(p, lds, m0, uniform(tile), M);
 }
 
 // 256 x 256 tiles, those from p.whole on as two 128 x 256 halves each.
-template <int WL>
-__global__ __launch_bounds__(256) void w8a8_deep_mix_kernel(W8A8Params p) {
+template <int WL, bool WIDE>
+__device__ __forceinline__ void w8a8_deep_mix_entry(const W8A8Params& p) {
   constexpr int L0 = W8A8DeepCfg<8, 8, 2, WL>::LDS, L1 = W8A8DeepCfg<4, 8, 3, WL>::LDS;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[L0 > L1 ? L0 : L1];
   tl_mark(p.tl, p.tl_cap, 0);  // diagnostics build: workgroup start
@@ -242,21 +248,31 @@ __global__ __launch_bounds__(256) void w8a8_deep_mix_kernel(W8A8Params p) {
   if (id < p.whole) {
     deep_tile_of(deep_order(id, p.whole), p.m_chunks, p.n_tiles, mc, tile);
     const int m0 = uniform(mc) * 256;
-    if (m0 < M) w8a8_deep_body<8, 8, 2, WL>(p, lds, m0, uniform(tile), M);
+    if (m0 < M) w8a8_deep_body<8, 8, 2, WL, WIDE>(p, lds, m0, uniform(tile), M);
   } else {
     const int idx = deep_order(id - p.whole, 2 * (p.m_chunks * p.n_tiles - p.whole));
     deep_tile_of(p.whole + idx / 2, p.m_chunks, p.n_tiles, mc, tile);
     const int m0 = uniform(mc) * 256 + (idx & 1) * 128;
-    if (m0 < M) w8a8_deep_body<4, 8, 3, WL>(p, lds, m0, uniform(tile), M);
+    if (m0 < M) w8a8_deep_body<4, 8, 3, WL, WIDE>(p, lds, m0, uniform(tile), M);
   }
 }
+
+template <int FM, int FN, int NSL, int WL>
+__global__ __launch_bounds__(256) void w8a8_deep_kernel(W8A8Params p) { w8a8_deep_entry<FM, FN, NSL, WL, false>(p); }
+template <int WL>
+__global__ __launch_bounds__(256) void w8a8_deep_mix_kernel(W8A8Params p) { w8a8_deep_mix_entry<WL, false>(p); }
+template <int FM, int FN, int NSL, int WL>
+__global__ __launch_bounds__(256) void w8a8_deep_wide_kernel(W8A8Params p) { w8a8_deep_entry<FM, FN, NSL, WL, true>(p); }
+template <int WL>
+__global__ __launch_bounds__(256) void w8a8_deep_mix_wide_kernel(W8A8Params p) { w8a8_deep_mix_entry<WL, true>(p); }
 
 // Tiles of the dispatch (api_w8a8.hip prices them), in order of the rows they are for.
 enum DeepTile { kDeep64, kDeep128, kDeep128Pair, kDeepMix, kDeepTiles };
 constexpr int kDeepRows[kDeepTiles] = {64, 128, 128, 256};       // token rows
 constexpr int kDeepChannels[kDeepTiles] = {128, 128, 128, 256};  // channels
 
-// Defined in the instantiation unit: the kernel of a tile for a weight layout, or null.
-const void* w8a8_deep_fn(int tile, int layout);
+// Defined in the instantiation unit: the kernel of a tile for a weight layout (`wide`: the one for rows
+// that span more than 4 GiB within a tile), or null.
+const void* w8a8_deep_fn(int tile, int layout, bool wide = false);
 
 }  // namespace specq

@@ -73,16 +73,19 @@ def test_many_rows_grouped_and_nonfinite_rows():
         assert torch.equal(o.view(torch.int16), ref.view(torch.int16))
 
 
-def test_many_rows_over_wide_strides():
-    """Activation rows that span more than 2 GiB within a tile: every row is read where it lies."""
-    M, N, Kd, ld = 700, 4096, 4096, 12 << 20
-    note(f"w4a16 many rows M={M} lda={ld}")
-    a, wp, sc, _ = operands("packed", M, N, Kd, 128, seed=6)
+@pytest.mark.parametrize("layout, M, N, Kd, ld", [("packed", 700, 4096, 4096, 12 << 20), ("packed", 700, 4096, 4096, 17 << 20),
+                                                  ("u8", 385, 8192, 4096, 18 << 20), ("i32", 385, 8192, 4096, 40 << 20)])
+def test_many_rows_over_wide_strides(layout, M, N, Kd, ld):
+    """Activation rows that span more than 2 or 4 GiB within a tile: every row is read where it lies."""
+    note(f"w4a16 many rows {layout} M={M} N={N} lda={ld}")
+    a, wp, sc, _ = operands(layout, M, N, Kd, 128, seed=6)
     wide = torch.empty((M, ld), dtype=torch.float16, device=DEV)
     wide[:, :Kd] = a
     out, ck = K.w4a16_matmul(wide[:, :Kd], wp, sc, BLOCK_M=None)
     ref, _ = K.w4a16_matmul(a, wp, sc, BLOCK_M=128)
     torch.cuda.synchronize()
+    del wide
+    torch.cuda.empty_cache()
     assert "deep_kernel" in ck.name, ck.name
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
 

@@ -93,16 +93,33 @@ def test_plan_at_grid_tiles_of_many_rows():
     assert bool((out[active:] == 7.0).all())
 
 
-def test_many_rows_over_wide_strides():
-    """Activation rows that span more than 2 GiB within a tile: every row is read where it lies."""
-    M, N, Kd, ld = 193, 7001, 1104, 40 << 20
-    note(f"w8a8 many rows M={M} lda={ld}")
-    a, sa, wp, sw, w = operands("w8a8", M, N, Kd, seed=6)
+# (format, M, N, K, row stride in bytes, kernel): every tile height with a tile's rows spanning more than
+# 4 GiB, the 64-row one also within it, the mixed launch as whole tiles and as halves.
+WIDE = [
+    ("w8a8", 193, 7001, 1104, 40 << 20, "deep_kernel<2, 4, 3, 1>"),
+    ("w8a8", 193, 7001, 1104, 80 << 20, "deep_kernel<2, 4, 3, 1>"),
+    ("w8a8", 385, 7001, 1104, 40 << 20, "deep_kernel<4, 4, 4, 1>"),
+    ("w8a8", 641, 10001, 3088, 34 << 20, "deep_kernel<4, 4, 2, 1>"),
+    ("w8a8", 513, 20000, 2048, 20 << 20, "deep_mix_kernel<1>"),
+    ("w8a8", 1024, 8192, 1040, 34 << 20, "deep_mix_kernel<1>"),
+    ("w4a8", 193, 28673, 208, 40 << 20, "deep_kernel<4, 4, 2, 2>"),
+]
+
+
+@pytest.mark.parametrize("fmt, M, N, Kd, ld, name", WIDE)
+def test_many_rows_over_wide_strides(fmt, M, N, Kd, ld, name):
+    """Activation rows that span gigabytes within a tile (one token of each long sequence): every row is
+    read where it lies, far past the 32 bits of a buffer offset."""
+    note(f"{fmt} many rows M={M} N={N} K={Kd} lda={ld}")
+    a, sa, wp, sw, w = operands(fmt, M, N, Kd, seed=6)
     wide = torch.empty((M, ld), dtype=torch.int8, device=DEV)
     wide[:, :Kd] = a
-    out, ck = K.w8a8_matmul(wide[:, :Kd], sa, wp, sw, BLOCK_M=None)
+    mm = K.w8a8_matmul if fmt == "w8a8" else K.w4a8_matmul
+    out, ck = mm(wide[:, :Kd], sa, wp, sw, BLOCK_M=None)
     torch.cuda.synchronize()
-    assert "deep_kernel<2, 4, 3, 1>" in ck.name, ck.name
+    del wide
+    torch.cuda.empty_cache()
+    assert name in ck.name, ck.name
     assert torch.equal(out.view(torch.int16), formula(a, sa, w, sw).view(torch.int16)), ck.name
 
 
