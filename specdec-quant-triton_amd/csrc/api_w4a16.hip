@@ -299,7 +299,8 @@ int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, in
   const int BM = mt * 16, BN = 64 * rw;
   cfg->ws_partials = cfg->splits > 1 ? align_up((size_t)cfg->m_chunks * cfg->n_tiles * cfg->splits * BM * BN * 4, 256) : 0;
   cfg->ws_counters = cfg->splits > 1 ? kCounterBytes : 0;
-  SPECQ_REQUIRE((int64_t)cfg->m_chunks * cfg->n_tiles <= kMaxCounters, SPECQ_ENOTSUP,
+  // The many-row kernel hands nothing over and has no counters.
+  SPECQ_REQUIRE(family == kW4Deep || (int64_t)cfg->m_chunks * cfg->n_tiles <= kMaxCounters, SPECQ_ENOTSUP,
                 "w4a16: %d x %d tiles exceed the counter region", cfg->m_chunks, cfg->n_tiles);
   if (family == kW4Deep) {
     w4_deep_launch(cfg);
@@ -374,7 +375,7 @@ int w4_group_config(int layout, int m_grid, int n_members, const int* N, int K, 
   cfg->ws_partials = cfg->splits > 1 ? align_up((size_t)cfg->m_chunks * tiles * cfg->splits * BM * BN * 4, 256) : 0;
   cfg->ws_counters = cfg->splits > 1 ? kCounterBytes : 0;
   if (cfg->family == kW4Deep) w4_deep_launch(cfg);
-  SPECQ_REQUIRE((int64_t)cfg->m_chunks * tiles <= kMaxCounters, SPECQ_ENOTSUP,
+  SPECQ_REQUIRE(cfg->family == kW4Deep || (int64_t)cfg->m_chunks * tiles <= kMaxCounters, SPECQ_ENOTSUP,
                 "w4a16_grouped: %d x %d tiles exceed the counter region", cfg->m_chunks, tiles);
   return SPECQ_OK;
 }

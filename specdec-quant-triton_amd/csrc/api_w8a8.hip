@@ -666,7 +666,8 @@ int w8a8_group_config(int layout, int m_grid, const W8A8Group& grp, int K, int b
   cfg->n_tiles = tiles;
   cfg->ws_partials =
       cfg->splits > 1 ? align_up((size_t)cfg->m_chunks * tiles * cfg->splits * (cfg->mt * 16) * cfg->bn * 4, 256) : 0;
-  SPECQ_REQUIRE((int64_t)cfg->m_chunks * tiles <= kMaxCounters, SPECQ_ENOTSUP,
+  // The many-row kernel hands nothing over and has no counters.
+  SPECQ_REQUIRE(cfg->family == kDeep || (int64_t)cfg->m_chunks * tiles <= kMaxCounters, SPECQ_ENOTSUP,
                 "w8a8: %d x %d tiles exceed the counter region", cfg->m_chunks, tiles);
   return SPECQ_OK;
 }

@@ -90,6 +90,26 @@ def test_many_rows_over_wide_strides(layout, M, N, Kd, ld):
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
 
 
+@pytest.mark.parametrize("members", [1, 2])
+def test_many_rows_past_the_counter_region(members):
+    """More tiles than there are split counters: the many-row kernel uses none."""
+    M, N, Kd = 262500, 4096 // members, 4096
+    note(f"w4a16 many rows M={M} members={members}")
+    a = torch.randn((M, Kd), device=DEV, generator=torch.Generator(device=DEV).manual_seed(8)).half()
+    ops = [operands("packed", 1, N, Kd, 128, seed=80 + i) for i in range(members)]
+    if members == 1:
+        out, ck = K.w4a16_matmul(a, *ops[0][1:3], BLOCK_M=None, split_k=4)
+        outs = [out]
+    else:
+        outs, ck = K.w4a16_matmul_grouped(a, [o[1:3] for o in ops], split_k=4)
+    torch.cuda.synchronize()
+    assert "deep_kernel" in ck.name, ck.name
+    for o, op in zip(outs, ops):
+        for rows in (slice(0, 300), slice(M - 300, M)):
+            ref, _ = K.w4a16_matmul(a[rows], *op[1:3], BLOCK_M=128, split_k=4)
+            assert torch.equal(o[rows].view(torch.int16), ref.view(torch.int16)), rows
+
+
 @pytest.mark.parametrize("block_m", [80, 96, 112, 128, 144, 160])
 @pytest.mark.parametrize("layout, rows", [("packed", 1), ("packed", 161), ("u8", 17), ("i32", 40)])
 def test_several_chunks_of_the_streaming_kernel(block_m, layout, rows):

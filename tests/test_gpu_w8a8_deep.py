@@ -123,6 +123,22 @@ def test_many_rows_over_wide_strides(fmt, M, N, Kd, ld, name):
     assert torch.equal(out.view(torch.int16), formula(a, sa, w, sw).view(torch.int16)), ck.name
 
 
+@pytest.mark.parametrize("M, Ns", [(37500, (14336, 14336)), (70100, (5120, 5120, 5120))])
+def test_many_rows_past_the_counter_region(M, Ns):
+    """Grouped launches of more tiles than the split counters: the many-row kernel uses none."""
+    Kd = 256
+    note(f"w4a8 grouped many rows M={M} N={Ns} K={Kd}")
+    ops = [operands("w4a8", M, N, Kd, seed=40 + i) for i, N in enumerate(Ns)]
+    a, sa = ops[0][:2]
+    outs, ck = K.w8a8_matmul_grouped(a, sa, [(o[2], o[3]) for o in ops], BLOCK_M=None)
+    torch.cuda.synchronize()
+    assert "deep_kernel<4, 4, 2, 2>" in ck.name, ck.name
+    for o, op in zip(outs, ops):
+        for rows in (slice(0, 300), slice(M // 2, M // 2 + 300), slice(M - 300, M)):
+            ref = formula(a[rows], sa[rows], op[4], op[3])
+            assert torch.equal(o[rows].view(torch.int16), ref.view(torch.int16)), rows
+
+
 @pytest.mark.parametrize("block_m", [48, 64, 128, 208, 304])
 @pytest.mark.parametrize("block_n, split_k", [(64, 1), (64, 3), (128, 1), (128, 4)])
 def test_several_chunks_of_the_streaming_kernel(block_m, block_n, split_k):
