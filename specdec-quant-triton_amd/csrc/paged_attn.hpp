@@ -401,11 +401,15 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, uint8_t (&r
     kv_base_v = (int64_t)pg * p.s_kp + (int64_t)tk * p.s_ko + (int64_t)kvh * p.s_kh;
     sc_base_v = ((int64_t)pg * p.s_sp + (int64_t)tk * p.s_so + (int64_t)kvh * p.s_sh) * (int64_t)sizeof(ST);
   }
-  // One query chunk: no other program reads these K/V bytes, and keeping them out of L2 leaves the
-  // lines of scales there, which the sequence's KV heads share (B = 32, one token, context 8192 116 ->
-  // 111 us, 4096 63.6 -> 60.8; B = 1, q_len 5, context 65536 45.1 -> 42.6).  Several query chunks read
-  // them again from L2 (2 x 256 tokens at context 4096: 70.0 us, and 71.7 kept out of it).
-  const bool read_once = p.n_qc == 1;
+  // One query chunk and D = 128: no other program reads these K/V lines, and keeping them out of L2
+  // leaves the lines of scales there, which the sequence's KV heads share.  Measured in a graph, us, kept ->
+  // not, on one cache replayed and (in brackets) on enough caches that none is found in the memory-side
+  // cache: B = 8, 9 tokens, context 4096 30.8 -> 29.5 (30.8 -> 30.0); B = 32, one token, context 4096 60.5
+  // -> 61.0 (64.0 -> 60.9), up to 8192 96.6 -> 94.9 (99.3 -> 95.3); B = 1, 5 tokens, context 65536 42.5 ->
+  // 43.4 (47.3 -> 44.5).  At D = 64 two KV heads' programs read halves of one line, and both need it: H = 16,
+  // H_KV = 4, B = 32, one token, up to 4096 22.9 -> 24.9 (23.9 -> 25.5).  Several query chunks read the lines
+  // again from L2 (2 x 256 tokens at context 4096: 70.0 us, and 71.7 kept out of it).
+  const bool read_once = D == 128 && p.n_qc == 1;
   // Issue the DMAs of chunk `it` into ring slot SL.  K/V granules of chunks past the wave's
   // last or on a page outside the pool, and of tokens at or past kv_end, are out of range
   // (zeros); their scales read a fixed valid address.
