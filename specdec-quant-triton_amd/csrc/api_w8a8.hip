@@ -356,6 +356,19 @@ int w8a8_deep_grid(const W8A8Cfg& cfg, int* whole) {
   return *whole + 2 * (total - *whole);
 }
 
+// Weights of a streaming launch stay in L2 where its M-chunks run together on one XCD (units that are
+// no multiple of 8 are interleaved, w8a8_ws.hpp).  In chunk-major order a chunk reads them a round of
+// workgroups after the one before, and keeping them gains only where one layer's weights are replayed
+// from the memory-side cache.  Non-temporal -> kept, us, over distinct weights and (in brackets) on one:
+// N = 10000, K = 3072, M = 128 15.2 -> 13.5 (13.4 -> 11.8), M = 100 14.7 -> 12.9; N = 5000, K = 3088, M = 100
+// 11.9 -> 10.9; but N = 4096, K = 14336, M = 128 23.5 -> 24.3 (24.7 -> 21.5), M = 288 38.0 -> 39.3 (39.0 -> 37.0).
+// One chunk reads them once (N = 28672, K = 4096, M = 72: 22.4, and 23.7 kept).
+void w8a8_keep(W8A8Cfg* cfg, bool plan_mode) {
+  cfg->keep = cfg->family == kWs && !plan_mode && cfg->m_chunks > 1 && cfg->n_tiles * cfg->splits % 8 != 0 &&
+              w8a8_ws_keeps(cfg->mt, cfg->bnsel, cfg->layout);
+  if (cfg->family == kWs) cfg->fn = ws_fn(cfg->bnsel, cfg->layout, cfg->mt, cfg->keep);
+}
+
 // Resolve the kernel and its tiles.  `vec` is the operand alignment (16 when unknown),
 // `layout` 0 = row-major weight, 1 = packed fragments.  `streaming`: no many-row tile (the answer is
 // one that explicit BLOCK_M, BLOCK_N and split_k name again).
@@ -450,10 +463,7 @@ int w8a8_config(int layout, int m_grid, int N, int K, int block_m, int block_n, 
       }
       fn = w8a8_rk_fn(bnsel, layout);
     } else {
-      // Weights that several M-chunks read stay in L2; with one chunk they are read once and do not
-      // (N = 28672, K = 4096, M = 72: 22.4 us, and 23.7 kept).
-      cfg->keep = !plan_mode && m_grid > mt * 16 && w8a8_ws_keeps(mt, bnsel, layout);
-      fn = ws_fn(bnsel, layout, mt, cfg->keep);
+      fn = ws_fn(bnsel, layout, mt, false);
     }
   }
   if (family == kLegacy) {
@@ -510,6 +520,7 @@ int w8a8_config(int layout, int m_grid, int N, int K, int block_m, int block_n, 
   cfg->k_range = k_range;
   cfg->ws_partials = splits > 1 ? align_up((size_t)cfg->m_chunks * cfg->n_tiles * splits * BM * BN * 4, 256) : 0;
   cfg->ws_counters = splits > 1 ? kCounterBytes : 0;
+  w8a8_keep(cfg, plan_mode);
   SPECQ_REQUIRE((int64_t)cfg->m_chunks * cfg->n_tiles <= kMaxCounters, SPECQ_ENOTSUP,
                 "w8a8: %d x %d tiles exceed the counter region", cfg->m_chunks, cfg->n_tiles);
   return SPECQ_OK;
@@ -666,6 +677,7 @@ int w8a8_group_config(int layout, int m_grid, const W8A8Group& grp, int K, int b
   cfg->n_tiles = tiles;
   cfg->ws_partials =
       cfg->splits > 1 ? align_up((size_t)cfg->m_chunks * tiles * cfg->splits * (cfg->mt * 16) * cfg->bn * 4, 256) : 0;
+  w8a8_keep(cfg, plan_mode);
   // The many-row kernel hands nothing over and has no counters.
   SPECQ_REQUIRE(cfg->family == kDeep || (int64_t)cfg->m_chunks * tiles <= kMaxCounters, SPECQ_ENOTSUP,
                 "w8a8: %d x %d tiles exceed the counter region", cfg->m_chunks, tiles);

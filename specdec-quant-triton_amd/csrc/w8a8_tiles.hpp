@@ -36,10 +36,9 @@ struct W8A8WsPick {
 };
 
 // Tiles of packed INT8 weights that automatic tiles run in several M-chunks (48 rows, 64 channels and
-// up) also come with weight loads that stay in L2 (w8a8_chunks_ws_kernel), for launches that have them
-// (non-temporal -> kept, us: N = 10000, K = 3072, M = 128 14.5 -> 12.8; N = 4096, K = 14336, M = 288 38.5 ->
-// 36.4, 517 53.2 -> 51.7; N = 3072, K = 8192, M = 256 20.9 -> 20.0).  INT4 fragments, half as long, do
-// not: N = 5120, K = 13824, M = 288 38.6 -> 40.3.
+// up) also come with weight loads that stay in L2 (w8a8_chunks_ws_kernel; w8a8_keep in api_w8a8.hip says
+// which launches take them).  INT4 fragments, half as long, do not: N = 5120, K = 13824, M = 288 38.6 ->
+// 40.3 us.
 constexpr bool w8a8_ws_keeps(int mt, int bnsel, int layout) { return mt >= 3 && bnsel >= 2 && layout == 1; }
 
 template <int MT, int BNSEL, int WL>

@@ -353,8 +353,8 @@ template <int MT, int RW, int KW, int S, int NSLOT, int NW, int WL>
 __global__ __launch_bounds__(NW * 64) void w8a8_ws_kernel(W8A8Params p) {
   w8a8_ws_entry<MT, RW, KW, S, NSLOT, NW, WL, false>(p);
 }
-// Eager launches of several M-chunks: the chunks of a channel tile share an XCD, and its L2 serves
-// the weight to all but the first.
+// Eager launches whose M-chunks of a channel tile run together on one XCD: its L2 serves the weight
+// to all but the first.
 template <int MT, int RW, int KW, int S, int NSLOT, int NW, int WL>
 __global__ __launch_bounds__(NW * 64) void w8a8_chunks_ws_kernel(W8A8Params p) {
   w8a8_ws_entry<MT, RW, KW, S, NSLOT, NW, WL, true>(p);
