@@ -343,9 +343,11 @@ int specq_silu_mul_quant_int8(const void* gate, int64_t ld_gate, const void* up,
  * of W4A8), 1 = W4A16 (layout in
  * `variant`), 2 = paged attention (D in `variant`, | 1 << 16 for fp32 K/V scales).  For the GEMMs, `variant` | 16 describes a
  * call made with a plan (m_grid is then grid_m_max); a plan-mode GEMM call with automatic
- * tiles reports the tiling it runs when the active M is m_grid.  kind 0, `variant` | 32: the best
- * tile that explicit block_m, block_n and split_k can name (an eager call of many rows with
- * automatic tiles may run one that they cannot: 64, 128 or 256 rows, block_n up to 256).
+ * tiles reports the tiling it runs when the active M is m_grid.  `variant` | 32 (GEMMs): the best
+ * tile that explicit block_m, block_n and split_k can name.  An eager call of many rows with
+ * automatic tiles may run one that they cannot: 64, 128 or 256 rows, block_n up to 256, reported without
+ * the flag; the same numbers given back run a streaming kernel (with the same results).  Its symbol
+ * is the one for rows that lie within 4 GiB in a tile.
  * ------------------------------------------------------------------------------------- */
 typedef struct specq_kernel_attrs {
   char name[160];          /* kernel symbol */

@@ -31,7 +31,7 @@ inline bool deep_wide(int rows, int64_t ld, int64_t len) { return (rows - 1) * l
 
 // Flag in the `variant` of a GEMM resource query: the call ran with a plan (tile rules differ).
 constexpr int kAttrsPlan = 16;
-// ... or the tiles are for an explicit request (W8A8: no many-row tile, which none names).
+// ... or the tiles are for an explicit request (no many-row tile, which none names).
 constexpr int kAttrsStreaming = 32;
 // Flag in the `variant` of an attention resource query: fp32 K/V scales (else fp16).
 constexpr int kAttrsScaleFp32 = 1 << 16;

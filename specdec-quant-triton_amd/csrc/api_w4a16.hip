@@ -236,7 +236,7 @@ bool w4_deep_wins(int M, int N, int K, int splits, int mt, int rw) {
 }
 
 int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, int split_k, bool plan_mode,
-              W4Cfg* cfg, bool allow_menu = true) {
+              W4Cfg* cfg, bool allow_menu = true, bool streaming = false) {
   SPECQ_REQUIRE(layout >= 0 && layout <= 2, SPECQ_EINVAL, "w4a16: unknown weight layout %d", layout);
   SPECQ_REQUIRE(m_grid >= 0 && N > 0 && K > 0, SPECQ_EINVAL, "w4a16: bad sizes M=%d N=%d K=%d", m_grid, N, K);
   SPECQ_REQUIRE(K % 128 == 0, SPECQ_ENOTSUP, "w4a16: K=%d must be a multiple of 128", K);
@@ -277,7 +277,7 @@ int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, in
     const int s_auto = std::min(split_k > 0 ? split_k : w4_auto_splits(N, nb), nb);
     const int s_eff = ceil_div(nb, ceil_div(nb, s_auto));
     w4_auto_tiles(m_grid, N, K, s_eff, block_n > 0 ? rw : 0, &mt, &rw);
-    deep = block_n <= 0 && g_w4a16_path.load() == 0 && w4_deep_wins(m_grid, N, K, s_eff, mt, rw);
+    deep = !streaming && block_n <= 0 && g_w4a16_path.load() == 0 && w4_deep_wins(m_grid, N, K, s_eff, mt, rw);
     if (deep) { mt = 8; rw = 2; }
   }
   // The LDS-staged kernel is the default at every depth (measured faster than the register
@@ -386,9 +386,9 @@ int w4a16_attrs(int layout, int m_grid, int N, int K, int block_m, int block_n, 
                 specq_kernel_attrs* out) {
   (void)num_warps;
   W4Cfg cfg;
-  const bool plan_mode = (layout & kAttrsPlan) != 0;
-  layout &= ~kAttrsPlan;
-  int rc = w4_config(layout, m_grid, N, K, block_m, block_n, split_k, plan_mode, &cfg);
+  const bool plan_mode = (layout & kAttrsPlan) != 0, streaming = (layout & kAttrsStreaming) != 0;
+  layout &= ~(kAttrsPlan | kAttrsStreaming);
+  int rc = w4_config(layout, m_grid, N, K, block_m, block_n, split_k, plan_mode, &cfg, true, streaming);
   if (rc) return rc;
   hipFuncAttributes fa;
   if (hipFuncGetAttributes(&fa, cfg.fn) != hipSuccess) return fail(SPECQ_EIO, "w4a16: hipFuncGetAttributes failed");

@@ -123,6 +123,8 @@ class KernelInfo:
 
     @property
     def config(self) -> dict:
+        """The tiles the call ran.  Given back as arguments they name the same kernel, except those of a
+        many-row kernel (block_n up to 256): these run a streaming kernel, with the same results."""
         a = self._get()
         return dict(block_m=a.block_m, block_n=a.block_n, num_warps=a.num_warps, split_k=a.split_k,
                     threads=a.threads, grid=a.grid)

@@ -774,6 +774,11 @@ def staircase_md(args) -> int:
     return 0
 
 
+def launch_key(M, ck):
+    """What names a launch: its kernel and tile (a many-row kernel's tile can equal a streaming one's)."""
+    return (M, ck.name, ck.config["block_m"], ck.config["block_n"], ck.config["split_k"])
+
+
 def staircase(args) -> int:
     """W8A8 (or, with --kind w4a16, W4A16) latency over M on the config-1 shapes: the library's
     tile choice at every M = 1..300 and fixed BLOCK_M at the staircase's edges."""
@@ -811,8 +816,7 @@ def staircase(args) -> int:
             for M in (range(1, 301) if bm is None else bounds):
                 # A fixed BLOCK_M that resolves to the same tiling as the automatic choice is the
                 # same launch: it reuses that timing instead of a second, noisy one.
-                cfg = K.KernelInfo(kid, 2 if w4 else 1, M, N, Kd, bm or 0, 0, 4, 0).config
-                key = (M, cfg["block_m"], cfg["block_n"], cfg["split_k"])
+                key = launch_key(M, K.KernelInfo(kid, 2 if w4 else 1, M, N, Kd, bm or 0, 0, 4, 0))
                 if key in timed:
                     row.setdefault(str(bm or "auto"), {})[M] = timed[key]
                     continue
@@ -843,14 +847,39 @@ TUNE_SHAPES = {"4096x4096": [(4096, 4096)], "1024x4096": [(1024, 4096)], "14336x
                "28672x4096": [(14336, 4096), (14336, 4096)]}
 
 
+MANY_ROW = None  # the tune candidate that no table entry can name: the many-row kernel
+
+
+def tune_candidates(info, w4, M):
+    """(candidates, the automatic one) of a tune step: tiles as (BLOCK_M, BLOCK_N, split_k), and MANY_ROW
+    where the cost model picks the many-row kernel.  info(block_m, block_n, streaming) is the KernelInfo of
+    a request, with `streaming` the best tile that an explicit request can name."""
+    auto = info(0, 0, True).config
+    reqs = [(0, 0)] + [(bm, 0) for bm in (16, 32, 64, 128)]
+    reqs += [(auto["block_m"], bn) for bn in ((64, 128) if w4 else (16, 32, 64, 128))]
+    if w4 and M > 144:
+        reqs.append((160, 0))  # the deepest W4A16 tile: M up to 320 in two chunks
+    cands = []
+    for bm, bn in reqs:
+        c = info(bm, bn, True).config
+        t = (c["block_m"], c["block_n"], c["split_k"])
+        if t not in cands:
+            cands.append(t)
+    if "deep" in info(0, 0, False).name:
+        return cands + [MANY_ROW], MANY_ROW
+    return cands, cands[0]
+
+
 def tune(args) -> int:
     """Measured tile table: for each config-1 launch shape and each step of M (M = 1..8, 9..16,
     then 16 rows at a time up to 300; timed at the step's first and last M, the mean of the
     two), the mean launch of every candidate
     tiling -- the automatic one, the reference's four BLOCK_M with the library's channel block
-    and split for that depth, and the automatic depth with every channel block -- each as a graph
+    and split for that depth, the automatic depth with every channel block, and the many-row kernel
+    where the cost model picks it -- each as a graph
     cycling over enough weight copies to stream from HBM.  Writes {kind: {shape: {rows16:
-    dict(best=[BLOCK_M, BLOCK_N, split_k], us, auto=[...], auto_us)}}} for `tune-emit`."""
+    dict(best=[BLOCK_M, BLOCK_N, split_k], us, auto=[...], auto_us)}}} for `tune-emit`; best and auto
+    are null for the many-row kernel, which no entry names (the step then has none)."""
     import torch
 
     if PKG not in sys.path:
@@ -891,7 +920,6 @@ def tune(args) -> int:
             sa = torch.rand((300,), device="cuda", generator=g) * 0.015 + 0.005
             outs = [torch.empty((300, N), dtype=torch.float16, device="cuda") for N, _ in members]
             kid = 1 if w4 else 0
-            bns = (64, 128) if w4 else (16, 32, 64, 128)
             # A grouped W4A16 launch runs its members' common split count: resolve tiles with it.
             gsk = K.w4a16_group_split([N for N, _ in members], Kd) if w4 else 0
             table = {}
@@ -902,20 +930,14 @@ def tune(args) -> int:
                 # them by the mean.
                 lo, M = (1, 8) if r == 0 else ((9, 16) if r == 1 else (16 * (r - 1) + 1, min(16 * r, 300)))
                 Ms = sorted({lo, M})
-                auto = K.KernelInfo(kid, 2 if w4 else 1, M, N_total, Kd, 0, 0, 4, gsk).config
-                reqs = [(None, None)] + [(bm, None) for bm in (16, 32, 64, 128)] + [(auto["block_m"], bn) for bn in bns]
-                if w4 and M > 144:
-                    reqs.append((160, None))  # the deepest W4A16 tile: M up to 320 in two chunks
-                cands = []
-                for bm, bn in reqs:
-                    c = K.KernelInfo(kid, 2 if w4 else 1, M, N_total, Kd, bm or 0, bn or 0, 4, gsk).config
-                    t = (c["block_m"], c["block_n"], c["split_k"])
-                    if t not in cands:
-                        cands.append(t)
+                cands, at = tune_candidates(
+                    lambda bm, bn, streaming: K.KernelInfo(kid, (2 if w4 else 1) | (32 if streaming else 0), M, N_total,
+                                                           Kd, bm, bn, 4, gsk), w4, M)
                 times, per_m = {}, {}
-                for bm, bn, sk in cands:
+                for cand in cands:
+                    bm, bn, sk = cand or (None, None, gsk)
                     tot = 0.0
-                    per_m[(bm, bn, sk)] = {}
+                    per_m[cand] = {}
                     for Mx in Ms:
                         def run(bm=bm, bn=bn, sk=sk, M=Mx):
                             for mem in weights:
@@ -927,10 +949,9 @@ def tune(args) -> int:
                                     K.w8a8_matmul_grouped(a[:M], sa[:M], mem, outs=o, BLOCK_M=bm, BLOCK_N=bn,
                                                           split_k=sk)
                         t = min(_graph_us(run, copies, reps=4), _graph_us(run, copies, reps=4))
-                        per_m[(bm, bn, sk)][Mx] = t
+                        per_m[cand][Mx] = t
                         tot += t
-                    times[(bm, bn, sk)] = tot / len(Ms)
-                at = (auto["block_m"], auto["block_n"], auto["split_k"])
+                    times[cand] = tot / len(Ms)
                 # The tile whose worst ratio to the fastest at each measured M of the step is
                 # smallest; the automatic tile unless that worst ratio is measurably better (2 %).
                 fastest = {Mx: min(per_m[c][Mx] for c in cands) for Mx in Ms}
@@ -938,11 +959,11 @@ def tune(args) -> int:
                 best = min(cands, key=lambda c: (regret[c], times[c]))
                 if regret[best] > regret[at] - 0.02:
                     best = at
-                print(f"[tune] {kind} {sname} step {r}: {list(best)}", flush=True)
-                table[r] = dict(best=list(best), us=round(times[best], 3), auto=list(at), auto_us=round(times[at], 3),
+                print(f"[tune] {kind} {sname} step {r}: {best}", flush=True)
+                table[r] = dict(best=best, us=round(times[best], 3), auto=at, auto_us=round(times[at], 3),
                                 regret=round(regret[best], 4), auto_regret=round(regret[at], 4),
-                                candidates={f"{b}x{n}s{k}": {str(m): round(t, 3) for m, t in per_m[(b, n, k)].items()}
-                                            for (b, n, k) in cands})
+                                candidates={f"{c[0]}x{c[1]}s{c[2]}" if c else "many-row":
+                                            {str(m): round(t, 3) for m, t in per_m[c].items()} for c in cands})
             res[kind][sname] = table
             print(f"[tune] {kind} {sname}: " + ", ".join(f"{r}:{table[r]['best']}" for r in table), flush=True)
             del weights
@@ -975,6 +996,8 @@ def tune_emit(args) -> int:
         for sname, table in shapes.items():
             N, Kd = (int(x) for x in sname.split("x"))
             for r in sorted(table, key=int):
+                if table[r]["best"] is MANY_ROW:
+                    continue  # no entry: the library's prices choose
                 bm, bn, sk = table[r]["best"]
                 lines.append(f"    {{{kid}, {N}, {Kd}, {int(r)}, {bm}, {bn}, {sk}}},")
                 n += 1
@@ -997,7 +1020,7 @@ def tune_md(args) -> int:
             print("|---|---|---|---|---|---|---|")
             for r in sorted(table, key=int):
                 e = table[r]
-                fmt = lambda t: f"{t[0]} x {t[1]}, {t[2]}"  # noqa: E731
+                fmt = lambda t: f"{t[0]} x {t[1]}, {t[2]}" if t else "many-row"  # noqa: E731
                 ri = int(r)
                 rng = "1-8" if ri == 0 else ("9-16" if ri == 1 else f"{16 * ri - 15}-{min(16 * ri, 300)}")
                 print(f"| {r} ({rng}) | {fmt(e['auto'])} | {e['auto_us']:.2f} | {fmt(e['best'])} | "

@@ -122,3 +122,14 @@ def test_several_chunks_of_the_streaming_kernel(block_m, layout, rows):
     torch.cuda.synchronize()
     assert "chunks_ws_kernel" in ck.name and "w4a16_ws_kernel" in ck64.name, (ck.name, ck64.name)
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16)), ck.name
+
+
+@pytest.mark.parametrize("kind, variant, M, N, Kd", [(0, 1, 513, 20000, 2048), (0, 2, 700, 10001, 3088), (1, 2, 1024, 4096, 4096)])
+def test_streaming_tile_of_a_many_row_shape_names_itself(kind, variant, M, N, Kd):
+    """`variant` | 32: a tile whose numbers, given back, ask for the same kernel."""
+    note(f"attrs kind={kind} variant={variant} M={M} N={N} K={Kd}")
+    assert "deep_" in K.KernelInfo(kind, variant, M, N, Kd, 0, 0, 4, 0).name
+    ck = K.KernelInfo(kind, variant | 32, M, N, Kd, 0, 0, 4, 0)
+    c = ck.config
+    again = K.KernelInfo(kind, variant, M, N, Kd, c["block_m"], c["block_n"], 4, c["split_k"])
+    assert "ws_kernel" in ck.name and ck.name == again.name and ck.config == again.config

@@ -285,3 +285,44 @@ def test_grid_markdown_tables():
     res = {(B, k, q): dict(us=float(B + k + q), frac=0.5) for B in (1, 2) for k in (0, 1) for q in ({k + 1, 1})}
     md = grids.attention_grid_md(res, 1024)
     assert "| 2 | 3.0 | 5.0 / 4.0 |" in md and "50.0 %" in md
+
+
+class _Info:
+    """KernelInfo of a library whose automatic tile is the many-row kernel's past 128 rows."""
+
+    def __init__(self, M, bm, bn, streaming):
+        deep = not streaming and not bm and not bn and M > 128
+        self.name = "w8a8_deep_kernel<2, 4, 3, 1>" if deep else "w8a8_ws_kernel<4>"
+        self.config = dict(block_m=64 if deep else bm or min(-(-M // 16) * 16, 304), block_n=bn or 128, split_k=1)
+
+
+@pytest.mark.parametrize("M", [72, 300])
+def test_tune_times_the_many_row_kernel_as_itself(M):
+    from specq import profiling as P
+    cands, auto = P.tune_candidates(lambda bm, bn, streaming: _Info(M, bm, bn, streaming), False, M)
+    rows = min(-(-M // 16) * 16, 304)
+    assert cands[0] == (rows, 128, 1) and (rows, 16, 1) in cands and (64, 128, 1) in cands
+    assert auto == ((rows, 128, 1) if M <= 128 else P.MANY_ROW) and auto in cands
+    assert len(set(cands)) == len(cands)
+
+
+def test_tune_emit_leaves_the_many_row_kernel_to_the_prices(tmp_path):
+    import argparse
+    import json
+
+    from specq import profiling as P
+    row = dict(us=1.0, auto=None, auto_us=1.0)
+    src = tmp_path / "t.json"
+    src.write_text(json.dumps({"w8a8": {"4096x4096": {"18": dict(row, best=None), "5": dict(row, best=[80, 64, 2])}}}))
+    out = tmp_path / "t.hpp"
+    P.tune_emit(argparse.Namespace(json=str(src), out=str(out)))
+    assert re.findall(r"\{0, .*?\}", out.read_text()) == ["{0, 4096, 4096, 5, 80, 64, 2}"]
+    assert "kTunedTileCount = 1" in out.read_text()
+    P.tune_md(argparse.Namespace(json=str(src)))
+
+
+def test_staircase_times_two_kernels_of_one_tile_apart():
+    from specq import profiling as P
+    deep, ws = _Info(300, 0, 0, False), _Info(300, 64, 128, False)
+    assert deep.config == ws.config and P.launch_key(300, deep) != P.launch_key(300, ws)
+    assert P.launch_key(300, ws) == P.launch_key(300, _Info(300, 64, 128, True))
