@@ -48,11 +48,8 @@ __device__ __forceinline__ void w4a16_deep_entry(W4A16Params p) {
 
   int mc, tile;
   deep_tile_of(deep_order((int)blockIdx.x, p.m_chunks * p.n_tiles), p.m_chunks, p.n_tiles, mc, tile);
-  int M = p.M;
-  if (p.plan != nullptr) M = min(max(p.plan[0], 0), p.m_grid);
-  M = uniform(M);
-  const int m0 = uniform(mc) * BM;
-  if (m0 >= M) return;
+  const int M = p.M, m0 = uniform(mc) * BM;
+  if (m0 >= M) return;  // the grid may cover more rows than there are
   const int ltile = w4_select_member(p, uniform(tile));
   const int lane = lane_id(), wv = uniform(wave_id()), g = lane >> 4, r = lane & 15;
   const int h = wv >> 2, w = wv & 3, wm = w & 1, wn = w >> 1;

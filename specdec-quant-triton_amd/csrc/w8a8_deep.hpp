@@ -62,9 +62,10 @@ struct W8A8DeepCfg {
 // The scalar arithmetic of that between the MFMAs costs 5 % (MLP block of M = 2048, hidden 4096, 14336
 // channels: 366 -> 383 us) and a branch in one kernel its registers, so it is a kernel of its own.
 template <int FM, int FN, int NSL, int WL, bool WIDE>
-__device__ __forceinline__ void w8a8_deep_body(W8A8Params p, uint8_t* lds, int m0, int tile, int M) {
+__device__ __forceinline__ void w8a8_deep_body(W8A8Params p, uint8_t* lds, int m0, int tile) {
   using C = W8A8DeepCfg<FM, FN, NSL, WL>;
   constexpr int BM = C::BM, BN = C::BN, FB = C::FB;
+  const int M = p.M;
   const int ltile = w8a8_select_member(p, tile);
   const int lane = lane_id(), w = uniform(wave_id()), g = lane >> 4, r = lane & 15;
   const int wm = w & 1, wn = w >> 1;
@@ -222,19 +223,14 @@ __device__ __forceinline__ void w8a8_deep_body(W8A8Params p, uint8_t* lds, int m
   tl_mark_drained(p.tl, p.tl_cap, 4);  // ... and completed
 }
 
-// Active rows.
-__device__ __forceinline__ int w8a8_deep_rows(const W8A8Params& p) {
-  return uniform(p.plan != nullptr ? min(max(p.plan[0], 0), p.m_grid) : p.M);
-}
-
 template <int FM, int FN, int NSL, int WL, bool WIDE>
 __device__ __forceinline__ void w8a8_deep_entry(const W8A8Params& p) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[W8A8DeepCfg<FM, FN, NSL, WL>::LDS];
   tl_mark(p.tl, p.tl_cap, 0);  // diagnostics build: workgroup start
   int mc, tile;
   deep_tile_of(deep_order((int)blockIdx.x, p.m_chunks * p.n_tiles), p.m_chunks, p.n_tiles, mc, tile);
-  const int M = w8a8_deep_rows(p), m0 = uniform(mc) * (32 * FM);
-  if (m0 < M) w8a8_deep_body<FM, FN, NSL, WL, WIDE>(p, lds, m0, uniform(tile), M);
+  const int m0 = uniform(mc) * (32 * FM);
+  if (m0 < p.M) w8a8_deep_body<FM, FN, NSL, WL, WIDE>(p, lds, m0, uniform(tile));  // the grid may cover more rows
 }
 
 // 256 x 256 tiles, those from p.whole on as two 128 x 256 halves each.
@@ -243,17 +239,17 @@ __device__ __forceinline__ void w8a8_deep_mix_entry(const W8A8Params& p) {
   constexpr int L0 = W8A8DeepCfg<8, 8, 2, WL>::LDS, L1 = W8A8DeepCfg<4, 8, 3, WL>::LDS;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[L0 > L1 ? L0 : L1];
   tl_mark(p.tl, p.tl_cap, 0);  // diagnostics build: workgroup start
-  const int M = w8a8_deep_rows(p), id = (int)blockIdx.x;
+  const int id = (int)blockIdx.x;
   int mc, tile;
   if (id < p.whole) {
     deep_tile_of(deep_order(id, p.whole), p.m_chunks, p.n_tiles, mc, tile);
     const int m0 = uniform(mc) * 256;
-    if (m0 < M) w8a8_deep_body<8, 8, 2, WL, WIDE>(p, lds, m0, uniform(tile), M);
+    if (m0 < p.M) w8a8_deep_body<8, 8, 2, WL, WIDE>(p, lds, m0, uniform(tile));
   } else {
     const int idx = deep_order(id - p.whole, 2 * (p.m_chunks * p.n_tiles - p.whole));
     deep_tile_of(p.whole + idx / 2, p.m_chunks, p.n_tiles, mc, tile);
     const int m0 = uniform(mc) * 256 + (idx & 1) * 128;
-    if (m0 < M) w8a8_deep_body<4, 8, 3, WL, WIDE>(p, lds, m0, uniform(tile), M);
+    if (m0 < p.M) w8a8_deep_body<4, 8, 3, WL, WIDE>(p, lds, m0, uniform(tile));
   }
 }
 
