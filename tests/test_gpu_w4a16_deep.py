@@ -58,6 +58,21 @@ def test_many_rows_bits_of_the_streaming_kernel(layout, M, N, Kd, group, split_k
     assert bool(((ws.double() - ref).abs() <= ref.abs() * 2.0 ** -11 + mag * Kd * 2.0 ** -24 + 1e-7).all())
 
 
+@pytest.mark.parametrize("M", [1, 129, 400])
+def test_many_rows_of_a_larger_grid(M):
+    """grid_m_max without a plan: the launch covers rows that there are not, whose workgroups end at once.
+    (No rows at all: an empty tensor has a null pointer, which the library refuses.)"""
+    note(f"w4a16 many rows M={M} grid_m_max=1024")
+    a, wp, sc, _ = operands("packed", M, 4096, 4096, 128, seed=10)
+    out = torch.full((1024, 4096), 7.0, dtype=torch.float16, device=DEV)
+    _, ck = K.w4a16_matmul(a[:M], wp, sc, out=out[:M], BLOCK_M=None, grid_m_max=1024)
+    torch.cuda.synchronize()
+    assert "deep_kernel" in ck.name, ck.name
+    ref, _ = K.w4a16_matmul(a[:M], wp, sc, BLOCK_M=64)
+    assert torch.equal(out[:M].view(torch.int16), ref.view(torch.int16))
+    assert bool((out[M:] == 7.0).all())
+
+
 def test_many_rows_grouped_and_nonfinite_rows():
     """Grouped members of unequal width; an activation row with Inf and NaN leaves the other rows alone."""
     M, Kd, Ns = 1020, 4096, (2048, 1030, 900)

@@ -64,6 +64,44 @@ def test_many_rows_bit_exact(fmt, M, N, Kd, name):
     assert bool((big[M:] == 7.0).all()) and bool((big[:, N:] == 7.0).all()), "stored past M or N"
 
 
+# Every tile, the mixed kernel's halves among them, at output rows that lanes store 16 bytes at a time:
+# contiguous ones, and padded ones whose last pieces are stored value by value.
+@pytest.mark.parametrize("fmt, M, N, Kd, name", [
+    ("w8a8", 150, 10000, 3088, "deep_kernel<2, 4, 3, 1>"),
+    ("w8a8", 385, 7000, 1104, "deep_kernel<4, 4, 4, 1>"),
+    ("w8a8", 641, 10000, 3088, "deep_kernel<4, 4, 2, 1>"),
+    ("w8a8", 1281, 10000, 3088, "deep_mix_kernel<1>"),
+    ("w8a8", 1023, 8184, 1040, "deep_mix_kernel<1>"),   # halves only
+    ("w4a8", 700, 10000, 3088, "deep_kernel<4, 4, 2, 2>"),
+])
+@pytest.mark.parametrize("odd", [0, 1, 5])
+def test_many_rows_aligned_output_rows(fmt, M, N, Kd, name, odd):
+    N -= odd
+    note(f"{fmt} many rows, aligned output rows M={M} N={N} K={Kd}")
+    a, sa, wp, sw, w = operands(fmt, M, N, Kd, seed=M + 1)
+    mm = K.w8a8_matmul if fmt == "w8a8" else K.w4a8_matmul
+    big = torch.full((M + 3, N + odd + (8 if odd else 0)), 7.0, dtype=torch.float16, device=DEV)
+    _, ck = mm(a, sa, wp, sw, out=big[:M, :N], BLOCK_M=None)
+    torch.cuda.synchronize()
+    assert name in ck.name and big.stride(0) % 8 == 0, (ck.name, big.stride(0))
+    assert torch.equal(big[:M, :N].view(torch.int16), formula(a, sa, w, sw).view(torch.int16)), ck.name
+    assert bool((big[M:] == 7.0).all()) and bool((big[:, N:] == 7.0).all()), "stored past M or N"
+
+
+@pytest.mark.parametrize("M", [1, 129, 400])
+def test_many_rows_of_a_larger_grid(M):
+    """grid_m_max without a plan: the launch covers rows that there are not, whose workgroups end at once.
+    (No rows at all: an empty tensor has a null pointer, which the library refuses.)"""
+    note(f"many rows M={M} grid_m_max=1281")
+    a, sa, wp, sw, w = operands("w8a8", M, 10000, 3088, seed=9)
+    out = torch.full((1281, 10000), 7.0, dtype=torch.float16, device=DEV)
+    _, ck = K.w8a8_matmul(a[:M], sa[:M], wp, sw, out=out[:M], BLOCK_M=None, grid_m_max=1281)
+    torch.cuda.synchronize()
+    assert "deep_mix_kernel<1>" in ck.name, ck.name
+    assert torch.equal(out[:M].view(torch.int16), formula(a[:M], sa[:M], w, sw).view(torch.int16))
+    assert bool((out[M:] == 7.0).all())
+
+
 def test_many_rows_grouped_members():
     """Members whose widths are no whole tiles, one below a tile, on a strided activation."""
     M, Kd, Ns = 1400, 1104, (7001, 40, 5000, 3000)
