@@ -329,23 +329,72 @@ double w8a8_stream_price(int M, int N, int K, double wb, int mt, int sel, int s,
   return t;
 }
 
-// The many-row tile of an eager call, or -1 where the streaming tile (mt, sel, s) is priced lower.
-// Both sides of the line, measured (us, streaming / many-row): N = 10240, K = 3072: M = 72 12.1 /
-// 13.9; N = 10000, K = 3072: M = 100 15.7 / 15.3, 192 19.7 / 13.3, 300 24.4 / 18.2; N = 3072, K = 8192: M = 256 22.0 / 24.7,
-// 517 32.0 / 26.0; N = K = 4096: M = 517 22.9 / 21.1, 1024 31.7 / 22.6; N = 28672, K = 4096: M = 517
-// 93 / 88, 1024 174 / 120, 2048 376 / 218; N = 4096, K = 14336: M = 517 53.9 / 56.8, 2048 144 / 101;
-// INT4 weights, N = 27648, K = 5120: M = 144 34.8 / 38.8, 256 55.3 / 40.0, 1024 206 / 131.
+// The same two prices where the weights come from memory, as each layer's do in a model (the ones above
+// were fitted on one layer's, which the memory-side cache holds): the many-row kernel's few chunks in
+// flight then wait for them, the more the fewer M-chunks share them.  Fitted over distinct weights to
+// 490 shapes of 130-2048 rows x 300-28672 channels x K 256-14336, 3 to 9 % rms; what output rows that are
+// not 16-byte aligned cost both kernels (1.55 us per million outputs) is left out of both.
+struct DeepCold {
+  double start, out;           // us, and us per million outputs
+  double fill, chunk, weight;  // what rows that there are not save and one M-chunk costs of the time per chunk
+                               // of K; us per million weight bytes
+  double full, part[3];        // us per chunk of K: a full round, and a last one by the workgroups per CU
+                               // (mixed: halves, whole tiles)
+};
+constexpr DeepCold kDeepCold[kDeepTiles] = {{4.35, 0.37, 0.45, 0.70, 0.019, 0.63, {0.35, 0.60}},
+                                            {6.0, 0.69, 0.42, 0.20, 0.0, 0.57, {0.46}},
+                                            {5.3, 0.35, 0.14, 0.18, 0.0, 0.94, {0.75, 0.90}},
+                                            {10.5, 0.11, 0.36, 0.06, 0.0, 1.73, {0.73, 1.52}}};
+constexpr DeepCold kDeepColdInt4 = {5.3, 0.25, 0.0, 0.15, 0.0, 1.04, {0.71, 0.80, 1.12}};
+
+double w8a8_deep_cold(int tile, int layout, int M, int N, int K, int cus) {
+  const DeepCold& c = layout == 2 ? kDeepColdInt4 : kDeepCold[tile];
+  const int m_chunks = ceil_div(M, kDeepRows[tile]);
+  const int occ = tile == kDeep128 || tile == kDeepMix ? 1 : (layout == 2 ? 3 : 2);  // workgroups per CU
+  const int64_t tiles = (int64_t)m_chunks * ceil_div(N, kDeepChannels[tile]), slots = (int64_t)cus * occ;
+  const int64_t rest = tiles % slots;
+  double per = c.full * (tiles / slots);
+  if (rest > 0) per += c.part[tile == kDeepMix ? (2 * rest > cus ? 1 : 0) : (rest - 1) / cus];
+  const double rows = (double)M / ((double)m_chunks * kDeepRows[tile]);
+  return c.start + c.out * 1e-6 * M * N + c.weight * 1e-6 * N * K * (layout == 2 ? 0.5 : 1.0) +
+         per * ceil_div(K, 128) * (1 - c.fill * (1 - rows) + c.chunk / m_chunks);
+}
+
+double w8a8_stream_cold(int M, int N, int K, double wb, int mt, int sel, int s, int cus) {
+  const int chunks = ceil_div(ceil_div(M, 16), mt), rows = mt * 16;
+  const int rounds = ceil_div(ceil_div(N, bn_of_sel(sel)) * s * chunks, cus);
+  double t = 4.05 + rounds * ((sel == 3 ? 0.046 : 0.0) + 0.0018 * rows) * (4 * ceil_div(K, 256)) / s +
+             0.88e-6 * M * N + 0.027e-6 * N * wb * K;
+  if (s > 1) t += 1.9 + 0.375e-6 * s * rows * chunks * N * 8;
+  return t;
+}
+
+// The many-row tile of an eager call, or -1 where the streaming tile (mt, sel, s) is priced lower, or
+// clearly lower over distinct weights (by more than 6 %, what the two prices err by).  Of those shapes, the
+// INT8 ones that the first comparison alone made slower over distinct weights by more than 5 % were 31 of
+// 302 (to 0.80 times the speed), with both 13 (0.88); INT4 7 of 189 (0.79), with both 3 (0.91).  Both sides of
+// the line, us over distinct weights and in brackets on one, streaming / many-row: N = 10000, K = 3072: M = 192
+// 15.0 / 15.8 (13.8 / 13.2), 300 19.2 / 18.5 (19.8 / 18.2); N = 3072, K = 8192: M = 256 21.1 / 29.7 (21.4 /
+// 24.1), 517 29.4 / 29.1 (31.2 / 26.5); N = K = 4096: M = 288 14.5 / 16.8 (14.4 / 14.4), 517 21.9 / 20.3 (23.3 /
+// 20.5), 1024 30.6 / 24.3 (32.6 / 24.0); N = K = 8192: M = 256 29.3 / 32.2 (29.5 / 27.8), 512 45.5 / 42.1 (46.5 /
+// 40.4); N = 28672, K = 4096: M = 517 90 / 107 (90 / 98), 1024 171 / 119 (171 / 111), 2048 334 / 222 (332 / 210);
+// N = 4096, K = 14336: M = 512 48.3 / 49.5 (49.7 / 43.1), 2048 137 / 108 (137 / 102); INT4 weights: N = 13824, K =
+// 5120, M = 256 29.1 / 36.6 (30.7 / 30.7); N = 27648, K = 5120: M = 144 31.9 / 41.1 (34.0 / 37.5), 256 51.6 / 43.1 (51.7 /
+// 39.7), 1024 195 / 135 (195 / 124).
 int w8a8_deep_tile(int layout, int M, int N, int K, int mt, int sel, int s) {
   if (M <= 128 || layout == 0) return -1;
   const int cus = device_cus();
-  double best = w8a8_stream_price(M, N, K, layout == 2 ? 0.5 : 1.0, mt, sel, s, cus);
+  const double wb = layout == 2 ? 0.5 : 1.0;
+  double best = w8a8_stream_price(M, N, K, wb, mt, sel, s, cus);
   int tile = -1;
   for (int i = 0; i < kDeepTiles; ++i) {
     if (w8a8_deep_fn(i, layout) == nullptr) continue;
     const double t = w8a8_deep_price(i, layout, M, N, K, cus);
     if (t < best) { best = t; tile = i; }
   }
-  return tile;
+  if (tile < 0) return -1;
+  const double stream = w8a8_stream_cold(M, N, K, wb, mt, sel, s, cus);
+  return w8a8_deep_cold(tile, layout, M, N, K, cus) <= 1.06 * stream ? tile : -1;
 }
 
 // Grid of a many-row launch and, of the mixed one, its whole tiles: every full round of them, and
