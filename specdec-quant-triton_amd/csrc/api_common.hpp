@@ -26,8 +26,10 @@ inline int fail(int code, const char* what) {
     }                                  \
   } while (0)
 
-// Whether a many-row tile's rows, ld bytes apart and len bytes long, reach past the 4 GiB of a buffer resource.
-inline bool deep_wide(int rows, int64_t ld, int64_t len) { return (rows - 1) * ld + len > 0xFFFFFFFFll; }
+// Whether a tile's rows, ld bytes apart and len bytes long, reach past `limit`: the 4 GiB of a buffer
+// resource for the many-row kernels, and 2 GiB for the streaming ones, whose masked loads lie there.
+inline bool rows_wide(int rows, int64_t ld, int64_t len, int64_t limit) { return (rows - 1) * ld + len > limit; }
+constexpr int64_t kDeepSpan = 0xFFFFFFFFll, kStreamSpan = 0x7FFFFFFFll;
 
 // Flag in the `variant` of a GEMM resource query: the call ran with a plan (tile rules differ).
 constexpr int kAttrsPlan = 16;

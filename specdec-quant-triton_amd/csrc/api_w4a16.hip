@@ -235,8 +235,9 @@ bool w4_deep_wins(int M, int N, int K, int splits, int mt, int rw) {
   return deep < 0.83 * ws;
 }
 
+// `streaming`: no many-row kernel; `wide`: always that one (rows that the others' offsets do not reach).
 int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, int split_k, bool plan_mode,
-              W4Cfg* cfg, bool allow_menu = true, bool streaming = false) {
+              W4Cfg* cfg, bool allow_menu = true, bool streaming = false, bool wide = false) {
   SPECQ_REQUIRE(layout >= 0 && layout <= 2, SPECQ_EINVAL, "w4a16: unknown weight layout %d", layout);
   SPECQ_REQUIRE(m_grid >= 0 && N > 0 && K > 0, SPECQ_EINVAL, "w4a16: bad sizes M=%d N=%d K=%d", m_grid, N, K);
   SPECQ_REQUIRE(K % 128 == 0, SPECQ_ENOTSUP, "w4a16: K=%d must be a multiple of 128", K);
@@ -280,6 +281,7 @@ int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, in
     deep = !streaming && block_n <= 0 && g_w4a16_path.load() == 0 && w4_deep_wins(m_grid, N, K, s_eff, mt, rw);
     if (deep) { mt = 8; rw = 2; }
   }
+  if (wide) { deep = true; mt = 8; rw = 2; }
   // The LDS-staged kernel is the default at every depth (measured faster than the register
   // stream even for 16-row tiles on the Llama-3-8B linears); the register stream stays
   // selectable for tiles of up to 32 rows.
@@ -321,6 +323,13 @@ int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, in
   return SPECQ_OK;
 }
 
+// Whether an eager call's rows lie further apart than the streaming kernels' offsets reach: the many-row
+// kernel reads any, with the same bits and no workspace.
+bool w4_rows_wide(const W4Cfg& cfg, const int32_t* plan, int M, int64_t lda, int K) {
+  return plan == nullptr && (cfg.family == kW4Ws || cfg.family == kW4Rk) &&
+         rows_wide(std::min(cfg.mt * 16, M), lda * 2, K * (int64_t)2, kStreamSpan);
+}
+
 size_t w4_workspace(int m_grid, int N, int K, int block_m, int block_n, int split_k) {
   // The partial-tile region does not depend on the weight layout or kernel family; take the
   // larger of the eager and plan-mode token tilings.
@@ -357,11 +366,11 @@ int w4_group_splits(int n_members, const int* N, int K, int split_k) {
 // M, reading the active M on the device), every member with the common split count; each
 // member's channel tiles start a new tile, so the launch-wide tile count is the members' sum.
 int w4_group_config(int layout, int m_grid, int n_members, const int* N, int K, int block_m, int block_n,
-                    int splits, bool plan_mode, W4Cfg* cfg, int* tile_end) {
+                    int splits, bool plan_mode, W4Cfg* cfg, int* tile_end, bool wide = false) {
   int64_t n_total = 0;
   for (int g = 0; g < n_members; ++g) n_total += N[g];
   SPECQ_REQUIRE(n_total <= INT32_MAX, SPECQ_EINVAL, "w4a16_grouped: total N too large");
-  int rc = w4_config(layout, m_grid, (int)n_total, K, block_m, block_n, splits, plan_mode, cfg, false);
+  int rc = w4_config(layout, m_grid, (int)n_total, K, block_m, block_n, splits, plan_mode, cfg, false, false, wide);
   if (rc) return rc;
   const int BN = 64 * cfg->rw, BM = cfg->mt * 16;
   int tiles = 0;
@@ -452,6 +461,10 @@ extern "C" int specq_w4a16(const void* a, int64_t lda, const void* wq, int64_t l
   W4Cfg cfg;
   int rc = w4_config(wq_layout, m_grid, N, K, block_m, block_n, split_k, plan != nullptr, &cfg);
   if (rc) return rc;
+  if (w4_rows_wide(cfg, plan, M, lda, K)) {
+    rc = w4_config(wq_layout, m_grid, N, K, block_m, block_n, split_k, false, &cfg, false, false, true);
+    if (rc) return rc;
+  }
   const size_t need = cfg.ws_partials + cfg.ws_counters;
   SPECQ_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), SPECQ_ENOSPC,
                 "w4a16: workspace of %zu bytes required, %zu given", need, workspace ? workspace_bytes : 0);
@@ -473,7 +486,8 @@ extern "C" int specq_w4a16(const void* a, int64_t lda, const void* wq, int64_t l
     for (int e = 0; e < kW4PlanRows; ++e) pp.t[e] = cfg.plan_t[e];
     return launch(cfg.fn, cfg.grid, kW4WsThreads, 0, (hipStream_t)stream, &pp);
   }
-  if (cfg.family == kW4Deep && deep_wide(std::min(cfg.mt * 16, M), lda * 2, K * (int64_t)2)) cfg.fn = w4a16_deep_fn(wq_layout, true);
+  if (cfg.family == kW4Deep && rows_wide(std::min(cfg.mt * 16, M), lda * 2, K * (int64_t)2, kDeepSpan))
+    cfg.fn = w4a16_deep_fn(wq_layout, true);
   return launch(cfg.fn, cfg.grid, cfg.family == kW4Rk ? 256 : kW4WsThreads, 0, (hipStream_t)stream, &p);
 }
 
@@ -546,6 +560,10 @@ extern "C" int specq_w4a16_grouped(const void* a, int64_t lda, int n_members, co
   int rc = w4_group_config(wq_layout, m_grid, n_members, N, K, block_m, block_n, splits, plan != nullptr, &cfg,
                            tile_end);
   if (rc) return rc;
+  if (w4_rows_wide(cfg, plan, M, lda, K)) {
+    rc = w4_group_config(wq_layout, m_grid, n_members, N, K, block_m, block_n, splits, false, &cfg, tile_end, true);
+    if (rc) return rc;
+  }
   const size_t need = cfg.ws_partials + cfg.ws_counters;
   SPECQ_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), SPECQ_ENOSPC,
                 "w4a16_grouped: workspace of %zu bytes required, %zu given", need, workspace ? workspace_bytes : 0);
@@ -576,7 +594,8 @@ extern "C" int specq_w4a16_grouped(const void* a, int64_t lda, int n_members, co
     p.grp_ntiles16[g - 1] = on ? ceil_div(N[g], 16) : 0;
     p.grp_vec_store[g - 1] = on ? vec_ok(g) : 0;
   }
-  if (cfg.family == kW4Deep && deep_wide(std::min(cfg.mt * 16, M), lda * 2, K * (int64_t)2)) cfg.fn = w4a16_deep_fn(wq_layout, true);
+  if (cfg.family == kW4Deep && rows_wide(std::min(cfg.mt * 16, M), lda * 2, K * (int64_t)2, kDeepSpan))
+    cfg.fn = w4a16_deep_fn(wq_layout, true);
   return launch(cfg.fn, cfg.grid, cfg.family == kW4Rk ? 256 : kW4WsThreads, 0, (hipStream_t)stream, &p);
 }
 

@@ -418,6 +418,17 @@ void w8a8_keep(W8A8Cfg* cfg, bool plan_mode) {
   if (cfg->family == kWs) cfg->fn = ws_fn(cfg->bnsel, cfg->layout, cfg->mt, cfg->keep);
 }
 
+// The many-row tile `deep` for a launch of width N.
+void w8a8_set_deep(int deep, int layout, int m_grid, int N, int K, W8A8Cfg* cfg) {
+  cfg->family = kDeep; cfg->deep = deep; cfg->layout = layout; cfg->vec = 16; cfg->nw = 4; cfg->rw = 1;
+  cfg->fn = w8a8_deep_fn(deep, layout);
+  cfg->mt = kDeepRows[deep] / 16; cfg->bn = kDeepChannels[deep]; cfg->bnsel = 3;
+  cfg->n_tiles = ceil_div(N, cfg->bn);
+  cfg->m_chunks = ceil_div(m_grid, kDeepRows[deep]);
+  cfg->splits = 1; cfg->k_range = ceil_div(K, 256) * 256;
+  cfg->lds = cfg->ws_partials = cfg->ws_counters = 0;
+}
+
 // Resolve the kernel and its tiles.  `vec` is the operand alignment (16 when unknown),
 // `layout` 0 = row-major weight, 1 = packed fragments.  `streaming`: no many-row tile (the answer is
 // one that explicit BLOCK_M, BLOCK_N and split_k name again).
@@ -453,13 +464,7 @@ int w8a8_config(int layout, int m_grid, int N, int K, int block_m, int block_n, 
     const int deep = block_n <= 0 && split_k <= 0 && !streaming
                          ? w8a8_deep_tile(layout, m_grid, N, K, mt, joint_sel, joint_splits) : -1;
     if (deep >= 0) {
-      cfg->family = kDeep; cfg->deep = deep; cfg->layout = layout; cfg->vec = vec; cfg->nw = 4; cfg->rw = 1;
-      cfg->fn = w8a8_deep_fn(deep, layout);
-      cfg->mt = kDeepRows[deep] / 16; cfg->bn = kDeepChannels[deep]; cfg->bnsel = 3;
-      cfg->n_tiles = ceil_div(N, cfg->bn);
-      cfg->m_chunks = ceil_div(m_grid, kDeepRows[deep]);
-      cfg->splits = 1; cfg->k_range = ceil_div(K, 256) * 256;
-      cfg->lds = cfg->ws_partials = cfg->ws_counters = 0;
+      w8a8_set_deep(deep, layout, m_grid, N, K, cfg);
       return SPECQ_OK;
     }
   } else if (block_m > 0) {
@@ -763,6 +768,14 @@ int run_w8a8(int layout, const int8_t* a, int64_t lda, const W8A8Group& grp, con
   W8A8Cfg cfg;
   int rc = w8a8_group_config(layout, m_grid, grp, K, block_m, block_n, num_warps, split_k, vec, plan != nullptr, &cfg);
   if (rc) return rc;
+  // Rows further apart than the streaming kernels' offsets reach: a many-row kernel reads any (the sums
+  // are exact in either, and it needs no workspace).
+  if (layout != 0 && plan == nullptr && (cfg.family == kWs || cfg.family == kRk) &&
+      rows_wide(std::min(cfg.mt * 16, M), lda, K, kStreamSpan)) {
+    w8a8_set_deep(layout == 2 ? kDeep128Pair : kDeep64, layout, m_grid, grp.n_total(), K, &cfg);
+    cfg.n_tiles = 0;
+    for (int g = 0; g < grp.n; ++g) cfg.n_tiles += ceil_div(grp.N[g], cfg.bn);
+  }
   const size_t need = cfg.ws_partials + cfg.ws_counters;
   if (static_scratch) {
     SPECQ_REQUIRE(need <= SPECQ_NOALLOC_SCRATCH_BYTES, SPECQ_ENOSPC,
@@ -806,7 +819,7 @@ int run_w8a8(int layout, const int8_t* a, int64_t lda, const W8A8Group& grp, con
   int grid = cfg.family == kPlan ? cfg.plan_grid : chunked_grid(cfg.n_tiles * cfg.splits, cfg.m_chunks);
   if (cfg.family == kDeep) {
     grid = w8a8_deep_grid(cfg, &p.whole);
-    if (deep_wide(std::min(kDeepRows[cfg.deep], M), lda, K)) cfg.fn = w8a8_deep_fn(cfg.deep, layout, true);
+    if (rows_wide(std::min(kDeepRows[cfg.deep], M), lda, K, kDeepSpan)) cfg.fn = w8a8_deep_fn(cfg.deep, layout, true);
   }
   if (static_scratch && need) {
     int n_ctr = cfg.family == kPlan ? cfg.n_counters : cfg.m_chunks * cfg.n_tiles;

@@ -105,6 +105,30 @@ def test_many_rows_over_wide_strides(layout, M, N, Kd, ld):
     assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
 
 
+@pytest.mark.parametrize("layout, M, N, Kd, ld, kw", [
+    ("packed", 72, 4096, 4096, 17 << 20, {}),
+    ("packed", 300, 6144, 1408, 10 << 20, dict(split_k=3)),              # 2 GiB and an odd number of blocks
+    ("u8", 160, 1030, 1280, 16 << 20, dict(BLOCK_M=160, BLOCK_N=64)),
+    ("i32", 9, 1030, 1280, 160 << 20, {}),
+])
+def test_streaming_tiles_over_wide_strides(layout, M, N, Kd, ld, kw):
+    """Rows further apart than the streaming kernels' offsets reach run the many-row kernel; what lies
+    between the rows (NaN here) is not read."""
+    note(f"w4a16 wide strides {layout} M={M} N={N} lda={ld} {kw}")
+    a, wp, sc, _ = operands(layout, M, N, Kd, 128, seed=17)
+    wide = torch.full((M, ld), float("nan"), dtype=torch.float16, device=DEV)
+    wide[:, :Kd] = a
+    kw = dict(dict(BLOCK_M=None), **kw)
+    out, _ = K.w4a16_matmul(wide[:, :Kd], wp, sc, **kw)
+    outs, _ = K.w4a16_matmul_grouped(wide[:, :Kd], [(wp, sc), (wp, sc)], **kw)
+    ref, _ = K.w4a16_matmul(a, wp, sc, **kw)
+    torch.cuda.synchronize()
+    del wide
+    torch.cuda.empty_cache()
+    for o in (out, *outs):
+        assert torch.equal(o.view(torch.int16), ref.view(torch.int16))
+
+
 @pytest.mark.parametrize("members", [1, 2])
 def test_many_rows_past_the_counter_region(members):
     """More tiles than there are split counters: the many-row kernel uses none."""

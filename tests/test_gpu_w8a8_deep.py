@@ -161,6 +161,31 @@ def test_many_rows_over_wide_strides(fmt, M, N, Kd, ld, name):
     assert torch.equal(out.view(torch.int16), formula(a, sa, w, sw).view(torch.int16)), ck.name
 
 
+@pytest.mark.parametrize("fmt, M, N, Kd, ld, tile", [
+    ("w8a8", 256, 8192, 8192, 40 << 20, {}),                      # a streaming tile by its price
+    ("w8a8", 72, 4096, 4096, 64 << 20, {}),
+    ("w8a8", 9, 4096, 4096, 300 << 20, {}),                       # 16-row tiles
+    ("w8a8", 500, 3001, 1040, 20 << 20, dict(BLOCK_M=304)),       # explicit tiles, split K
+    ("w8a8", 300, 1030, 1296, 20 << 20, dict(BLOCK_M=208, BLOCK_N=64, split_k=3)),
+    ("w4a8", 144, 5120, 1040, 40 << 20, {}),
+])
+def test_streaming_tiles_over_wide_strides(fmt, M, N, Kd, ld, tile):
+    """Rows further apart than the streaming kernels' offsets reach run a many-row kernel."""
+    note(f"{fmt} wide strides M={M} N={N} K={Kd} lda={ld} {tile}")
+    a, sa, wp, sw, w = operands(fmt, M, N, Kd, seed=16)
+    wide = torch.empty((M, ld), dtype=torch.int8, device=DEV)
+    wide[:, :Kd] = a
+    mm = K.w8a8_matmul if fmt == "w8a8" else K.w4a8_matmul
+    out, _ = mm(wide[:, :Kd], sa, wp, sw, **dict(dict(BLOCK_M=None), **tile))
+    outs, _ = K.w8a8_matmul_grouped(wide[:, :Kd], sa, [(wp, sw), (wp, sw)], **dict(dict(BLOCK_M=None), **tile))
+    torch.cuda.synchronize()
+    del wide
+    torch.cuda.empty_cache()
+    ref = formula(a, sa, w, sw).view(torch.int16)
+    for o in (out, *outs):
+        assert torch.equal(o.view(torch.int16), ref)
+
+
 @pytest.mark.parametrize("M, Ns", [(37500, (14336, 14336)), (70100, (5120, 5120, 5120))])
 def test_many_rows_past_the_counter_region(M, Ns):
     """Grouped launches of more tiles than the split counters: the many-row kernel uses none."""
