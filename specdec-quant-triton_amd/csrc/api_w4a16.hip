@@ -220,10 +220,13 @@ void w4_deep_launch(W4Cfg* cfg) {
 // Whether an eager call of several K splits runs the many-row kernel rather than the streaming tile
 // (mt, rw), by measured prices (us).  Many-row: per round of workgroups a start and an end, 2.45 us
 // per pair of K blocks and 0.5 us per split.  Streaming: the model above, whose error past 512 rows
-// is a fifth, and the splits' partial tiles written and read back at 3 TB/s; together they come out
-// up to a sixth high (290 to 1500 rows of nine layers), which the line allows for.  Both sides of it,
-// measured (streaming / many-row): N = K = 4096: M = 512 40 / 46, 700 59 / 46, 1024 85 / 50; N = 4096,
-// K = 14336: M = 512 81 / 134, 1024 188 / 144, 2048 343 / 278; N = 6144, K = 4096: M = 1024 86 / 88.
+// is a fifth, and the splits' partial tiles written and read back at 3 TB/s; together they came out
+// up to a sixth high (290 to 1500 rows of nine layers), which the line allows for.  (Fitted before either
+// kernel kept its weights in L2: both are now up to a tenth faster than their price.)  Both sides of the
+// line, us over distinct weights and in brackets on one, streaming / many-row: N = K = 4096: M = 512
+// 41 / 46 (40 / 44), 700 56 / 46 (54 / 45), 1024 81 / 48 (79 / 49); N = 4096, K = 14336: M = 512 83 / 131 (80 /
+// 125), 700 122 / 129 (118 / 126), 1024 178 / 139 (176 / 136), 2048 332 / 275 (329 / 268); N = K = 5120: M = 1500
+// 131 / 101 (131 / 103); N = 6144, K = 4096: M = 1024 89 / 87 (86 / 83), left to the streaming kernel.
 bool w4_deep_wins(int M, int N, int K, int splits, int mt, int rw) {
   if (M <= 256 || splits <= 1) return false;
   const int cus = device_cus(), rows16 = ceil_div(M, 16);
@@ -309,9 +312,12 @@ int w4_config(int layout, int m_grid, int N, int K, int block_m, int block_n, in
   } else if (family == kW4Rk) {
     cfg->fn = w4a16_rk_fn(mt, rw, layout);
   } else {
-    // Weights that several M-chunks read stay in L2 (N = 4096, K = 14336: M = 512 81.5 -> 78.6 us;
-    // N = 28672, K = 4096: M = 288 79.2 -> 75.9, 1024 293 -> 288); with one chunk they are read once and
-    // do not (a layer's four launches at M = 72: 79 us, and 84 kept).
+    // Weights that several M-chunks read stay in L2.  Non-temporal -> kept, us, over distinct weights and
+    // (in brackets) on one: N = 3072, K = 8192, M = 400 39.6 -> 36.8 (40.6 -> 36.0); N = 6144, K = 4096, M = 400
+    // 36.5 -> 34.5 (37.7 -> 34.0); N = 4096, K = 14336, M = 700 127.9 -> 123.1 (129.2 -> 118.6), M = 400 74.8 ->
+    // 76.1 (77.0 -> 73.6); N = 28672, K = 4096, M = 288 80.7 -> 81.3 (81.6 -> 79.0); geometric mean of 26 shapes at
+    // 200 to 1024 rows 1.005 (1.037), -2.5 to +8 %.  With one chunk they are read once and do not (a
+    // layer's four launches at M = 72: 79 us, and 84 kept).
     cfg->keep = !plan_mode && cfg->m_chunks > 1 && mt >= kW4KeepMt;
     switch (layout) {
       case 0: cfg->fn = w4a16_ws_fn_l0(mt, rw, cfg->keep); break;

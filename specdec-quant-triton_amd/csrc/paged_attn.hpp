@@ -18,8 +18,9 @@
 //    a sequence filling the block table, at most 8192 tokens and at most 64 splits, and at
 //    least 256 tokens (384 once the block table holds 4096 tokens or more), the units spread
 //    evenly over the splits (attn_split_units).  It depends only on the block table's
-//    capacity and the number of active sequences, so a QPP=1 and a fused program, and an eager and a plan-mode call, cut
-//    a sequence at the same tokens, and the page ids of a split can be fetched before the
+//    capacity, the number of active sequences and the 64-row programs that their query tokens fill
+//    (attn_row_programs), so a QPP=1 and a fused program, and an eager and a plan-mode call, cut a
+//    sequence at the same tokens, and the page ids of a split can be fetched before the
 //    sequence's length is known.
 //  * Eight waves (two per SIMD, so one wave's MFMA and LDS latencies hide behind the other's
 //    arithmetic) take interleaved 16-token chunks of the split (chunk c, one page sub-tile,
@@ -840,8 +841,10 @@ __device__ __forceinline__ void paged_attn_body(const AttnParams& p, uint8_t (&r
   // Row weights of the splits, exp2(m_s - max) / l (l summed in split order), in LDS (the rings,
   // no longer read).  All (m, l) pairs are fetched by all threads, in flight together, and every
   // row's thread then walks its splits in LDS: a row's thread fetching its own pairs beyond the
-  // first 16 splits waited for each load in turn (B = 1, q_len 5, context 65536, 31 splits: the
-  // launch's graph replay 59.9 -> 53.5 us; B = 8, q_len 9, context 4096, 4 splits: 37.0 -> 36.3).
+  // first 16 splits waited for each load in turn (per launch in a graph: B = 1, q_len 5, context 65536,
+  // 31 splits 49.7 -> 43.4 us; B = 1, q_len 9, 8192 tokens 32.4 -> 27.1; B = 8, q_len 9, context 4096, 4 splits
+  // 30.6 -> 30.0; 64-row programs, 2 x 64 tokens at context 4096 36.4 -> 35.0, although the RB = 4 program spills
+  // eight more registers around the wave merge).
   constexpr int WST = kAttnMergeMax + 1;  // row stride: the rows' threads walk different banks
   float* wts = reinterpret_cast<float*>(&ring0[0][0]);  // [ROWS][WST], m then the weight
   float* lst = reinterpret_cast<float*>(&ring1[0][0]);  // [ROWS][WST], l

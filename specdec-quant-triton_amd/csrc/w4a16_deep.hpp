@@ -12,13 +12,15 @@
 // K are summed one after the other by the same workgroup, in the order the streaming kernel's last
 // workgroup adds them, with nothing handed over.
 //
-// Measured (us, streaming -> here): M = 1024, N = K = 4096 85 -> 50, N = 4096, K = 14336 188 -> 144,
-// M = 1500, N = K = 5120 134 -> 106; with the weight loads kept in L2, where the other M-chunks of the
-// channel tile find them, instead of non-temporal, M = 1024, K = 14336 142 -> 134, 700 126 -> 117.  Unsplit layers stay with the streaming kernel, which runs them at
-// the same rate (0.75 to 0.85 PFLOP/s).  Copies without the dequantization, without the LDS reads and
-// without the DMAs ran within a few percent of the kernel.  Also tried: the next fragment
-// dequantized between the MFMAs of this one, wave priorities by stream and around the MFMAs, weights
-// two blocks ahead: no gain.
+// Measured (us over distinct weights, streaming -> here): M = 1024, N = K = 4096 81 -> 48, N = 4096, K =
+// 14336 178 -> 139, M = 1500, N = K = 5120 131 -> 101.  The weight loads stay in L2, where the other
+// M-chunks of the channel tile find them (M = 1024, K = 14336, on one layer's weights: 142 -> 134 from
+// non-temporal loads).  Unsplit layers stay with the streaming kernel, which runs them at the same rate
+// (0.75 to 0.85 PFLOP/s).  Counters at M = 1024, K = 14336: the matrix cores are busy 36 % of the launch;
+// a wave issues VALU work, mostly the dequantization, a quarter of its time (two waves a SIMD) and waits
+// 38 % of it for an issue slot and 28 % for memory and LDS (profiles/many_row_gemms_counters.md).  Also
+// tried: the next fragment dequantized between the MFMAs of this one, wave priorities by stream and
+// around the MFMAs, weights two blocks ahead: no gain.
 //
 //  * A stream walks its 128-wide K blocks, a block a chunk: the 256 bytes of each activation row
 //    land in one of the stream's two LDS slots by LDS DMA, 16-byte pieces XOR-swizzled by row;

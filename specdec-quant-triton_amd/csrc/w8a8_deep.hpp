@@ -11,10 +11,12 @@
 // fragments for 64 MFMAs, every byte of both operands crosses L2 -> CU once per 256 x 256 tile,
 // and 256 accumulator registers leave room for two sets of operands.
 //
-// Measured (us, streaming -> here; INT8 weights unless said): M = 2048, N = 28672, K = 4096 376 -> 218
-// (2.2 POPS; the same launch on all-zero operands takes a quarter less, so the clock under load is
-// most of what is left), N = 4096, K = 14336 144 -> 101; M = 1024, N = K = 4096 31.7 -> 22.6; INT4
-// weights, M = 1024, N = 27648, K = 5120 206 -> 131.  Also tried: 64-byte K steps in a ring twice as
+// Measured (us over distinct weights and, in brackets, on one; streaming -> here; INT8 weights unless
+// said): M = 2048, N = 28672, K = 4096 334 -> 222 (332 -> 210, 2.3 POPS), N = 4096, K = 14336 137 -> 108 (137 ->
+// 102); M = 1024, N = K = 4096 30.6 -> 24.3 (32.6 -> 24.0); INT4 weights, M = 1024, N = 27648, K = 5120 195 -> 135
+// (195 -> 124).  Counters at M = 2048: the matrix cores are busy 46 to 50 % of the launch, a wave waits 41 %
+// of its time for an issue slot and 17 % for memory, LDS and barriers, and the clock is 1.9 GHz under
+// this load (profiles/many_row_gemms_counters.md).  Also tried: 64-byte K steps in a ring twice as
 // deep (218 -> 264 and slower at every large tile), splits of K over workgroups for few tiles (slower
 // than the streaming kernel at M <= 517), 256 x 128 tiles (slower than 128 x 256).
 //
